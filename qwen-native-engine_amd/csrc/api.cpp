@@ -377,7 +377,10 @@ int qne_gemm(int kind, const void* w, const void* sz, int rows, int k, int group
         a.N = rows;
         a.K = k;
         a.group = kind == QNE_MAT_Q4 ? group : 64;
-        a.splits = qne::gemm_splits(kind, rows, k, a.group);
+        // up to 256 rows share one split count and form, so a row's sums do not depend on the call;
+        // longer calls would write a partial of every row per split and run as a prompt's pass
+        if (m > 256 && kind == QNE_MAT_Q4) a.row_tiles = (m + 63) / 64;
+        a.splits = qne::gemm_splits(kind, rows, k, a.group, a.row_tiles);
         a.epi = epilogue;
         a.y = y;
         a.y_stride = y_stride;

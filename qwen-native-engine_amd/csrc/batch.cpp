@@ -44,6 +44,7 @@ void rows_gemm(const DevMat& W, int n, float eps, uint8_t* frag, int norm, float
     a.K = W.k;
     a.group = W.group;
     a.splits = gemm_splits(W.kind, W.rows, W.k, W.group, row_tiles);
+    a.row_tiles = row_tiles;
     a.part = part;
     a.epi = epi;
     a.y = y;

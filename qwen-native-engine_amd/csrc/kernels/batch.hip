@@ -28,6 +28,7 @@
 #include "launch.hpp"
 #include "lds_dma.hpp"
 #include "operand.hpp"
+#include "q4_mfma.hpp"
 
 namespace qne {
 
@@ -35,31 +36,6 @@ namespace {
 
 using namespace lds_dma;
 
-
-typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-typedef float float16_t __attribute__((ext_vector_type(16)));
-
-// The 8 nibbles of a q4 word (nibble i at bits 4i: column 8j + i of word j) as exact f16 values, in
-// the order [q0, q4, q1, q5, q2, q6, q3, q7]: 0x6400 | q is the f16 1024 + q, and 0x6400 | (q << 4)
-// is 1024 + 16 q, so four and-or, one shift, two packed subtracts and two packed fmas (x / 16 - 64)
-// give all eight. The x operand of a q4 GEMM is staged in the same column order.
-__device__ __forceinline__ half8_t nibbles8(uint32_t v) {
-    typedef uint32_t u32;
-    const u32 v2 = v >> 8;
-    const u32 t0 = (v & 0x000F000Fu) | 0x64006400u;
-    const u32 t1 = (v & 0x00F000F0u) | 0x64006400u;
-    const u32 t2 = (v2 & 0x000F000Fu) | 0x64006400u;
-    const u32 t3 = (v2 & 0x00F000F0u) | 0x64006400u;
-    const half2_t k1024 = {(_Float16)1024.0f, (_Float16)1024.0f};
-    const half2_t k16 = {(_Float16)0.0625f, (_Float16)0.0625f};
-    const half2_t k64 = {(_Float16)-64.0f, (_Float16)-64.0f};
-    const half2_t h0 = __builtin_bit_cast(half2_t, t0) - k1024;
-    const half2_t h1 = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, t1), k16, k64);
-    const half2_t h2 = __builtin_bit_cast(half2_t, t2) - k1024;
-    const half2_t h3 = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, t3), k16, k64);
-    return half8_t{h0.x, h0.y, h1.x, h1.y, h2.x, h2.y, h3.x, h3.y};
-}
 __device__ __forceinline__ uint32_t pack_h2(float a, float b) {
     return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)a) | ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)b) << 16);
 }
@@ -107,8 +83,7 @@ __device__ __forceinline__ void wait_vm_upto(int n) {
 // Epilogues: partials (split-K, or an epilogue the GEMM does not apply); `direct` (one split: store
 // or residual add); `fuse` 1 (one split, SwiGLU): tiles [0, TW / 2) are gate rows and [TW / 2, TW)
 // the matching up rows (n_out further), and the workgroup writes silu(gate) * up and stages it as
-// the next GEMM's operand; `fuse` 2 (one split, store or residual add with the result staged as the
-// next GEMM's operand). Both compute exactly what k_gemm_reduce does with one split.
+// the next GEMM's operand, exactly as k_gemm_reduce does with one split.
 template <int KIND, int WAVES, int D, int DW, int CF>
 __global__ __launch_bounds__(64 * (WAVES + DW)) void k_gemm(const GemmArgs a) {
     constexpr int TW = WAVES * CF;                                  // 32-row W tiles per workgroup
@@ -326,51 +301,6 @@ __global__ __launch_bounds__(64 * (WAVES + DW)) void k_gemm(const GemmArgs a) {
                     store_through(d, a.epi == EPI_ACCUMULATE ? *d + v : v);
                 }
             }
-        }
-        return;
-    }
-    if (a.fuse == 2) {
-        // the tile through LDS ([row][column]) times the rows' 1 / rms, then every wave takes whole
-        // 64-column chunks of rows (lanes = columns): residual add or store, and the staged operand
-        constexpr int kOut = TW * 32;  // output columns of the workgroup
-        static_assert(kOut % kChunk == 0 && (kBM * kOut + kBM) * 4 <= D * kSlot, "fused epilogue tile");
-        float* so = sinv + kBM;  // [kBM][kOut]
-        if (computes) {
-#pragma unroll
-            for (int cf = 0; cf < CF; cf++) {
-                const int col = (w * CF + cf) * 32 + l32;
-#pragma unroll
-                for (int j = 0; j < 16; j++) {
-                    const int m = 8 * (j / 4) + 4 * hf + (j % 4);
-                    so[m * kOut + col] = acc[cf][0][j] * sinv[m];
-                    so[(32 + m) * kOut + col] = acc[cf][1][j] * sinv[32 + m];
-                }
-            }
-        }
-        __syncthreads();
-        if (!computes) return;
-        constexpr int nck = kOut / kChunk;
-        constexpr int kIt = kBM * nck / WAVES;  // (row, chunk) items per wave: item w + WAVES q
-        static_assert(kBM * nck % WAVES == 0, "fused epilogue items");
-        const size_t tile_bytes = (size_t)(a.n_out / kChunk) * kChunkBytes;
-        const int nrow = min(rows, kBM), col0 = blockIdx.x * kOut;
-        // every item's residual and gain loads in flight before the first is used
-        float hv[kIt], gv[kIt];
-#pragma unroll
-        for (int q = 0; q < kIt; q++) {
-            const int it = w + WAVES * q, r = it / nck, ch = it % nck, c = col0 + ch * kChunk + lane;
-            const bool live = r < nrow && col0 + ch * kChunk < a.n_out;  // else a whole chunk past the outputs
-            hv[q] = live && a.epi == EPI_ACCUMULATE ? a.y[(size_t)(kBM * mt + r) * a.y_stride + c] : 0.0f;
-            gv[q] = live && a.gain_out ? a.gain_out[c] : 1.0f;
-        }
-#pragma unroll
-        for (int q = 0; q < kIt; q++) {
-            const int it = w + WAVES * q, r = it / nck, ch = it % nck, c = col0 + ch * kChunk + lane;
-            if (r >= nrow || col0 + ch * kChunk >= a.n_out) continue;  // wave-uniform
-            const float g = so[r * kOut + ch * kChunk + lane];
-            const float v = a.epi == EPI_ACCUMULATE ? hv[q] + g : g;
-            if (a.y) store_through(a.y + (size_t)(kBM * mt + r) * a.y_stride + c, v);
-            emit_x(a.frag_out, tile_bytes, kBM * mt + r, c, v, gv[q], a.order_out, lane);
         }
         return;
     }
@@ -641,16 +571,14 @@ void launch_gemm(GemmArgs a, hipStream_t st) {
         launch_stage_x(a.x, a.x_stride, a.m, a.K, a.gain, a.kind == KIND_Q4 ? 1 : 0, a.frag, st);
         a.norm = a.gain ? 1 : 0;
     }
+    const bool wide = a.kind == KIND_Q4 && a.row_tiles > 1;
     const int waves = gemm_waves(a.kind, a.N);
     const dim3 grid((a.N + 32 * waves - 1) / (32 * waves), a.splits, a.mpad / kBM);
     // One row tile (a batched decode step): about one workgroup per CU, so 4 DMA waves beside the
     // 8 compute waves let the transfers overlap the computation (64 rows: gate_up 23.9 -> 22.4 us,
-    // LM head 222 -> 205 us). Several row tiles (a prefill pass): two 8-wave workgroups per CU
-    // (125 VGPRs in a 12-wave workgroup leave room for one). Measured and not kept for the prefill:
-    // 4 compute waves of 64 columns each (every A fragment read from LDS feeding two MFMAs), slower
-    // on every shape (gate_up 68 -> 108 us): each wave then issues 9 LDS DMAs per chunk instead of
-    // 5, and a DMA holds its wave for about the transfer time.
-    const bool dma_waves = a.mpad == kBM;
+    // LM head 222 -> 205 us). Several row tiles (calls of 65 to 256 rows, and f16 passes): two 8-wave
+    // workgroups per CU (125 VGPRs in a 12-wave workgroup leave room for one).
+    const bool dma_waves = a.mpad == kBM && !wide;
     // One split over several row tiles: the GEMM applies the SwiGLU, or the store / residual add,
     // and stages the output itself, with no partials and no reduce pass
     const bool one = a.fuse == 0 && a.kind == KIND_Q4 && !dma_waves && a.splits == 1 && !a.partials_only;
@@ -659,11 +587,13 @@ void launch_gemm(GemmArgs a, hipStream_t st) {
         (a.y || a.frag_out))
         a.fuse = 1;
     // store or residual add staged as the next operand (with a normed input its 1 / rms needs K <= 4096)
-    else if (one && a.epi != EPI_SWIGLU && a.frag_out && a.n_out == a.N && a.N % kChunk == 0 &&
+    else if (one && wide && a.epi != EPI_SWIGLU && a.frag_out && a.n_out == a.N && a.N % kChunk == 0 &&
              (a.epi == EPI_STORE || a.y) && (!a.norm || a.K <= 64 * kChunk))
         a.fuse = 2;
     a.direct = a.splits == 1 && a.epi != EPI_SWIGLU && !a.frag_out && !a.partials_only;
-    if (a.kind == KIND_Q4) {
+    if (wide) {
+        launch_gemm_wide(a, st);
+    } else if (a.kind == KIND_Q4) {
         // 3 chunk slots (77.6 KiB): deeper rings measured slower, and two workgroups fit a CU
         if (dma_waves) hipLaunchKernelGGL((k_gemm<KIND_Q4, 8, 3, 4, 1>), grid, dim3(768), 0, st, a);
         else hipLaunchKernelGGL((k_gemm<KIND_Q4, 8, 3, 0, 1>), grid, dim3(512), 0, st, a);

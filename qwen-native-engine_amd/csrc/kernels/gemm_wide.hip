@@ -1,0 +1,448 @@
+// The q4 GEMM of a pass over a prompt: many rows of x, y = x W^T.
+//
+// The batched step's GEMM (batch.hip) keeps one 64-row tile of x and streams W past it; over many
+// rows that form read every x fragment from LDS once per 32 columns and every scale and row sum once
+// per chunk, and left the matrix units idle for 70 % of the time. Here:
+//  - a wave computes 64 rows x 64 columns, so 18 KiB of LDS reads feed 32 MFMAs (17 KiB fed 16), and
+//    a weight is dequantised once per 64 rows;
+//  - the weights enter the matrix units as q - 8 and the zero points' share, sum over the chunks of
+//    s (8 - z) sum x, is the accumulators' first value: one small product on the bf16 matrix units
+//    (f32 operands as three bf16 terms, six products, to 2^-24), before the first chunk. A chunk then
+//    costs one fma per output value instead of two, and no row sums from LDS; the error against 64
+//    bits is 0.6 of what it was (the products no longer carry the zero points);
+//  - the epilogue stages the next GEMM's operand 16 bytes a lane.
+// A workgroup is 8 waves over 256 columns. 128 rows (KG = 1): 2 x 4 waves, every wave takes every
+// chunk. 64 rows (KG = 2): 4 waves across, and the two halves of the workgroup take the even and the
+// odd chunks; their sums meet in LDS at the end. The second form gives matrices with few columns twice
+// the workgroups at the same LDS traffic per MFMA. Which form a column runs in depends on the matrix
+// and the caller's fixed row count, never on the rows of the call, so a row's sums are added in the
+// same order in every call.
+// Measured (2048 rows, K = 2048): N = 12288 with its epilogue 261 -> 203 us (206 GFLOP of MFMA, 1.0
+// PFLOP/s; a loop of these MFMAs alone on such data reaches 1.85), N = 8224 210 -> 157 us, N = 2048
+// 62 -> 43 us; K = 6144, N = 2048 136 -> 109 us. What is left: a workgroup's start and end are ~12 us
+// with its CU's matrix units idle, and a chunk (1.7 us) spends a third of its time around the barrier.
+#include <algorithm>
+#include <type_traits>
+
+#include "../error.hpp"
+#include "common.hpp"
+#include "launch.hpp"
+#include "lds_dma.hpp"
+#include "operand.hpp"
+#include "q4_mfma.hpp"
+
+namespace qne {
+
+namespace {
+
+using namespace lds_dma;
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+
+// v as three bf16 terms (round to nearest: 27 bits in all, so the sum is v).
+struct Bf3 {
+    bf16x8_t t[3];
+    __device__ __forceinline__ void set(int i, float v) {
+        const __bf16 a = (__bf16)v;
+        const float r = v - (float)a;
+        const __bf16 b = (__bf16)r;
+        t[0][i] = a;
+        t[1][i] = b;
+        t[2][i] = (__bf16)(r - (float)b);
+    }
+};
+
+constexpr int kWideCols = 256;  // W rows (output columns) of a workgroup
+constexpr int kWideWaves = 8;
+constexpr int kWideRing = 3;    // slots: one computed, two in flight
+
+}  // namespace
+
+// LDS of a workgroup: the ring of slots (x of two (row tile | chunk) halves, 8 W tiles of 32 rows, their
+// scale / zero words), reused for the output tile; and the rows' 1 / rms.
+template <int KG>
+struct WideLds {
+    static constexpr int kRows = 128 / KG;
+    static constexpr int kX = 2 * 2 * kFragBytes;
+    static constexpr int kW = KG * 8 * 1024;
+    static constexpr int kSz = KG * 8 * 128;
+    static constexpr int kSlot = kX + kW + kSz;
+    static constexpr int kOutStride = kWideCols + 4;  // staged output rows, padded against bank conflicts
+    static constexpr int kRing = kWideRing * kSlot > kRows * kOutStride * 4 ? kWideRing * kSlot : kRows * kOutStride * 4;
+    __attribute__((aligned(16))) uint8_t ring[kRing];
+    float sinv[kRows];
+    float parts[512];                                 // partial sums of the rows' x^2
+};
+
+// Column tile bx, row tile bz (of 128 / KG rows), split by: chunks [by cps, (by + 1) cps).
+template <int KG>
+__device__ __forceinline__ void wide_tile(const GemmArgs& a, WideLds<KG>& lds, const int bx, const int by, const int bz) {
+    typedef WideLds<KG> L;
+    constexpr int kRows = L::kRows, kX = L::kX, kW = L::kW, kSlot = L::kSlot, kOutStride = L::kOutStride;
+    constexpr int kPer = 4 + KG + 1;                // DMAs of a wave per ring slot
+    uint8_t* const ring = lds.ring;
+    float* const sinv = lds.sinv;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int hf = lane >> 5, l32 = lane & 31;
+    const int half = w >> 2, nw = w & 3;            // half: row tile (KG 1) or chunk parity (KG 2)
+    const int nchunks = a.K / kChunk, cpg = a.group / kChunk, ngroups = nchunks / cpg;
+    const int c0 = by * a.cps, c1 = min(nchunks, c0 + a.cps);
+    const int iters = (c1 - c0 + KG - 1) / KG;
+    const int row0 = bz * kRows;
+    const int last_tile = a.mpad / kBM - 1;
+    const size_t tile_bytes = (size_t)nchunks * kChunkBytes;
+    // this wave's half of x: rows 64 half.. of the workgroup (a tile past the rows: the last one, not
+    // stored), or all its rows for every second chunk
+    const uint8_t* xtile = a.frag + (size_t)min(KG == 1 ? bz * 2 + half : bz, last_tile) * tile_bytes;
+    const int cfirst = c0 + (KG == 2 ? half : 0);   // this wave's first chunk
+    // first W row (= output column) of tile t; a SwiGLU's even tiles are gate rows, the odd ones the
+    // matching up rows, so a wave holds both factors of its 32 columns
+    auto wrow0 = [&](int t) -> int {
+        if (a.fuse == 1) return (t & 1 ? a.n_out : 0) + (bx * 4 + (t >> 1)) * 32;
+        return (bx * 8 + t) * 32;
+    };
+
+    // sources of this wave's DMAs: 4 KiB of its half's x, W tile w, its words
+    constexpr int kPieces = 2 * KG;                 // 16-byte pieces of a W row per slot
+    const int tile0 = min(wrow0(w), a.N - 1);       // past N: row N - 1, not stored
+    const uint8_t* wbase = (const uint8_t*)a.W + (size_t)tile0 * (a.K / 2);
+    const uint8_t* szbase = (const uint8_t*)a.SZT + (size_t)(tile0 >> 5) * ngroups * 128;
+    uint32_t woff[KG];
+    int wchunk[KG];                                 // the piece's chunk within the slot
+#pragma unroll
+    for (int u = 0; u < KG; u++) {
+        const int row = (64 / kPieces) * u + lane / kPieces;
+        int piece = lane % kPieces;
+        if (KG == 2) piece ^= (row >> 2) & 3;       // rows 4 apart on different banks
+        wchunk[u] = piece >> 1;
+        woff[u] = (uint32_t)(min(wrow0(w) + row, a.N - 1) - tile0) * (a.K / 2) + 16 * (piece & 1);
+    }
+    auto group = [&](int c) -> int { return cpg == 1 ? c : (int)((unsigned)c / (unsigned)cpg); };
+    // DMA u (of kPer) of slot j
+    const uint32_t ring_lds = lds_address(ring);
+    auto issue = [&](int j, int slot, int u) {
+        const uint32_t base = ring_lds + slot * kSlot;
+        const int c = c0 + KG * j;
+        if (u < 4) {
+            dma16_at(xtile + (size_t)min(c + (KG == 2 ? half : 0), c1 - 1) * kChunkBytes + 4096 * nw + 1024 * u, 16 * lane,
+                     base + 2 * kFragBytes * half + 4096 * nw + 1024 * u);
+        } else if (u < 4 + KG) {
+            if (KG == 1) dma16_at(wbase + (size_t)c * 32, woff[0], base + kX + 1024 * w);
+            else dma16_at(wbase, woff[u - 4] + min(c + wchunk[u - 4], c1 - 1) * 32, base + kX + KG * 1024 * w + 1024 * (u - 4));
+        } else if (lane < 8 * KG) {
+            if (KG == 1) dma16_at(szbase + (size_t)group(c) * 128, 16 * lane, base + kX + kW + 128 * w);
+            else dma16_at(szbase, (uint32_t)group(min(c + (lane >> 3), c1 - 1)) * 128 + 16 * (lane & 7), base + kX + kW + KG * 128 * w);
+        }
+    };
+    // acc's first value: sum over this wave's chunks of s (8 - z) sum x. The chunks are the contraction,
+    // 16 at a time; a batch's loads are in flight together, the first batch's (and the first sums of
+    // x^2) ahead of the first chunks' DMAs.
+    const int nmine = (c1 - cfirst + KG - 1) / KG;
+    const float* xsum = (const float*)(xtile + kXsumOff) + l32;
+    const uint32_t* szt[2];
+#pragma unroll
+    for (int t = 0; t < 2; t++) szt[t] = a.SZT + (size_t)(min(wrow0(2 * nw + t), a.N - 1) >> 5) * ngroups * 32 + l32;
+    float xv[2][8];
+    uint32_t sz[2][8];
+    auto load_sums = [&](int b) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int c = cfirst + KG * max(0, min(b + 8 * hf + i, nmine - 1)), g = group(min(c, c1 - 1));
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                xv[t][i] = xsum[(size_t)min(c, c1 - 1) * (kChunkBytes / 4) + 32 * t];
+                sz[t][i] = szt[t][(size_t)g * 32];
+            }
+        }
+    };
+    load_sums(0);
+    // A row's sum of x^2: thread t of the row's 4 KG takes the chunks t + 4 KG k (a batch of 64), and
+    // the tree below adds them in the order of row_inv_rms (a butterfly over 64 lanes, lane = chunk).
+    const bool norm = a.norm && (a.direct || a.fuse);
+    constexpr int TR = 4 * KG, KR = 64 / TR;
+    const int rr = threadIdx.x % kRows, tr = threadIdx.x / kRows;
+    const float* ssp = (const float*)(a.frag + (size_t)min((row0 + rr) / kBM, last_tile) * tile_bytes + kSsOff) + (rr & (kBM - 1));
+    float sq[KR];
+    if (norm) {
+#pragma unroll
+        for (int k = 0; k < KR; k++) {
+            const int c = tr + TR * k;
+            const float v = ssp[(size_t)min(c, nchunks - 1) * (kChunkBytes / 4)];
+            sq[k] = c < nchunks ? v : 0.0f;
+        }
+    }
+    for (int j = 0; j < min(kWideRing - 1, iters); j++)
+#pragma unroll
+        for (int u = 0; u < kPer; u++) issue(j, j, u);
+    if (norm) {
+        for (int c0n = 64; c0n < nchunks; c0n += 64)
+#pragma unroll
+            for (int k = 0; k < KR; k++) {
+                const int c = c0n + tr + TR * k;
+                const float v = ssp[(size_t)min(c, nchunks - 1) * (kChunkBytes / 4)];
+                sq[k] += c < nchunks ? v : 0.0f;
+            }
+#pragma unroll
+        for (int d = KR / 2; d >= 1; d >>= 1)
+#pragma unroll
+            for (int k = 0; k < d; k++) sq[k] += sq[k + d];
+        lds.parts[tr * kRows + rr] = sq[0];
+    }
+    float16_t acc[2][2] = {};
+    for (int b = 0; b < nmine; b += 16) {
+        Bf3 xa[2], wb[2];
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const bool live = b + 8 * hf + i < nmine;
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                xa[t].set(i, live ? xv[t][i] : 0.0f);
+                wb[t].set(i, live ? lo_h(sz[t][i]) * (8.0f - hi_h(sz[t][i])) : 0.0f);
+            }
+        }
+        if (b + 16 < nmine) load_sums(b + 16);
+#pragma unroll
+        for (int p = 2; p >= 0; p--)
+#pragma unroll
+            for (int q = 0; q <= p; q++)
+#pragma unroll
+                for (int cf = 0; cf < 2; cf++)
+#pragma unroll
+                    for (int rt = 0; rt < 2; rt++)
+                        acc[cf][rt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[rt].t[q], wb[cf].t[p - q], acc[cf][rt], 0, 0, 0);
+    }
+
+    // A chunk runs as two phases, one per 32-row tile, of four k-steps: the first dequantises the
+    // weights and keeps them for the second. The scaled sums of a phase are added during the next
+    // one, and the DMAs of a later slot go out between the steps, so the matrix unit has work
+    // throughout a phase. The empty asm statements pin each step's vector work to its step: left
+    // alone, the compiler gathers it at the end of the chunk and copies grp to keep it alive.
+    // Measured and not kept: the workgroup's second half one phase behind the first (5 % slower).
+    int slot = 0, next_slot = kWideRing - 1;
+    float16_t grp[2][2] = {};       // [column tile][row tile]
+    float sc[2] = {};
+    const int piece = KG == 1 ? hf : (2 * half + hf) ^ ((l32 >> 2) & 3);
+    auto chunk = [&](int j, auto sends) {
+        const uint8_t* xs = ring + slot * kSlot + 2 * kFragBytes * half;
+        const uint8_t* ws = ring + slot * kSlot + kX + 2 * nw * KG * 1024;
+        const uint8_t* wsz = ring + slot * kSlot + kX + kW + 2 * nw * KG * 128 + (KG == 2 ? 128 * half : 0) + 4 * l32;
+        uint4 wq[2];
+        uint32_t szw[2];
+        half8_t b[2][4];
+#pragma unroll
+        for (int cf = 0; cf < 2; cf++) wq[cf] = *(const uint4*)(ws + cf * KG * 1024 + (l32 * kPieces + piece) * 16);
+        half8_t ah = *(const half8_t*)(xs + frag_offset(0, 0, lane)), al = *(const half8_t*)(xs + kFragBytes + frag_offset(0, 0, lane));
+#pragma unroll
+        for (int cf = 0; cf < 2; cf++) szw[cf] = *(const uint32_t*)(wsz + cf * KG * 128);
+#pragma unroll
+        for (int p = 0; p < 8; p++) {
+            const int rt = p >> 2, s = p & 3, np = p + 1;
+            half8_t nh = ah, nl = al;
+            if (np < 8) {
+                nh = *(const half8_t*)(xs + frag_offset(np & 3, np >> 2, lane));
+                nl = *(const half8_t*)(xs + kFragBytes + frag_offset(np & 3, np >> 2, lane));
+            }
+            if (rt == 0) {
+#pragma unroll
+                for (int cf = 0; cf < 2; cf++) b[cf][s] = nibbles8_signed(s == 0 ? wq[cf].x : s == 1 ? wq[cf].y : s == 2 ? wq[cf].z : wq[cf].w);
+            }
+            const float16_t zero = {};
+#pragma unroll
+            for (int cf = 0; cf < 2; cf++) grp[cf][rt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, b[cf][s], s == 0 ? zero : grp[cf][rt], 0, 0, 0);
+#pragma unroll
+            for (int cf = 0; cf < 2; cf++) grp[cf][rt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, b[cf][s], grp[cf][rt], 0, 0, 0);
+            if (p == 4) {
+#pragma unroll
+                for (int cf = 0; cf < 2; cf++) sc[cf] = lo_h(szw[cf]);
+            }
+#pragma unroll
+            for (int cf = 0; cf < 2; cf++)
+#pragma unroll
+                for (int e = 4 * s; e < 4 * s + 4; e++) {
+                    float v = fmaf(sc[cf], grp[cf][1 - rt][e], acc[cf][1 - rt][e]);
+                    asm volatile("" : "+v"(v));
+                    acc[cf][1 - rt][e] = v;
+                }
+            if (sends && p < kPer) issue(j + kWideRing - 1, next_slot, p);
+            __builtin_amdgcn_sched_barrier(0);
+            ah = nh;
+            al = nl;
+        }
+        slot = slot + 1 == kWideRing ? 0 : slot + 1;
+        next_slot = next_slot + 1 == kWideRing ? 0 : next_slot + 1;
+    };
+    // A wave whose columns all lie past N only sends. At the barrier every part of slot j has landed,
+    // and every wave is done with slot j - 1.
+    const bool dead = wrow0(2 * nw) >= a.N;
+    for (int j = 0; j < iters - (kWideRing - 1); j++) {
+        wait_vm<kPer>();
+        __syncthreads();
+        if (dead) {
+#pragma unroll
+            for (int u = 0; u < kPer; u++) issue(j + kWideRing - 1, next_slot, u);
+            next_slot = next_slot + 1 == kWideRing ? 0 : next_slot + 1;
+        } else {
+            chunk(j, std::true_type());
+        }
+    }
+    if (iters > 1) {
+        wait_vm<kPer>();
+        __syncthreads();
+        if (!dead) chunk(iters - 2, std::false_type());
+    }
+    wait_vm<0>();
+    __syncthreads();
+    if (!dead && (KG == 1 || cfirst + KG * (iters - 1) < c1)) chunk(iters - 1, std::false_type());  // the odd half may have no last chunk
+    if (threadIdx.x < kRows) {
+        float inv = 1.0f;
+        if (norm) {
+            float t[TR];
+#pragma unroll
+            for (int k = 0; k < TR; k++) t[k] = lds.parts[k * kRows + threadIdx.x];
+#pragma unroll
+            for (int d = TR / 2; d >= 1; d >>= 1)
+#pragma unroll
+                for (int k = 0; k < d; k++) t[k] += t[k + d];
+            inv = 1.0f / sqrtf(t[0] / (float)a.K + a.eps);
+        }
+        sinv[threadIdx.x] = inv;
+    }
+#pragma unroll
+    for (int cf = 0; cf < 2; cf++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) acc[cf][1][e] = fmaf(sc[cf], grp[cf][1][e], acc[cf][1][e]);
+    __syncthreads();  // ring no longer read
+
+    // KG = 2: the halves' sums, even + odd chunks; each half then owns one 32-row tile
+    constexpr int RT = KG == 1 ? 2 : 1;
+    if (KG == 2) {
+        float* x = (float*)ring;  // [half's gift][nw][cf][e][lane]
+#pragma unroll
+        for (int cf = 0; cf < 2; cf++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) x[(((half * 4 + nw) * 2 + cf) * 16 + e) * 64 + lane] = half ? acc[cf][0][e] : acc[cf][1][e];
+        __syncthreads();
+#pragma unroll
+        for (int cf = 0; cf < 2; cf++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) {
+                const float o = x[((((1 - half) * 4 + nw) * 2 + cf) * 16 + e) * 64 + lane];
+                acc[cf][0][e] = half ? o + acc[cf][1][e] : acc[cf][0][e] + o;
+            }
+        __syncthreads();
+    }
+    const int rb = KG == 1 ? 64 * half : 32 * half;  // this wave's first row of the workgroup
+    if (!a.direct && !a.fuse) {  // split partials
+#pragma unroll
+        for (int cf = 0; cf < 2; cf++) {
+            const int n = wrow0(2 * nw + cf) + l32;
+            if (n >= a.N) continue;
+#pragma unroll
+            for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) {
+                    const int r = row0 + rb + 32 * rt + 8 * (e / 4) + 4 * hf + (e % 4);
+                    if (r < a.mpad) store_through(a.part + ((size_t)by * a.mpad + r) * a.N + n, acc[cf][rt][e]);
+                }
+        }
+        return;
+    }
+    // the epilogue in registers; with frag_out the values also go to LDS, [row][column]
+    float* so = (float*)ring;
+    if (a.fuse == 1) {
+        const int col = 32 * nw + l32, n = bx * 128 + col;
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) {
+                const int r = rb + 32 * rt + 8 * (e / 4) + 4 * hf + (e % 4);
+                const float v = silu(acc[0][rt][e] * sinv[r]) * (acc[1][rt][e] * sinv[r]);
+                if (a.y && row0 + r < a.m) store_through(a.y + (size_t)(row0 + r) * a.y_stride + n, v);
+                if (a.frag_out) so[r * kOutStride + col] = v;
+            }
+    } else {
+#pragma unroll
+        for (int cf = 0; cf < 2; cf++) {
+            const int n = wrow0(2 * nw + cf) + l32;
+            // the residual's loads all in flight before the first is used
+            float hv[RT][16];
+#pragma unroll
+            for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) {
+                    const int r = row0 + rb + 32 * rt + 8 * (e / 4) + 4 * hf + (e % 4);
+                    hv[rt][e] = a.epi == EPI_ACCUMULATE && n < a.N && r < a.m ? a.y[(size_t)r * a.y_stride + n] : 0.0f;
+                }
+#pragma unroll
+            for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) {
+                    const int r = rb + 32 * rt + 8 * (e / 4) + 4 * hf + (e % 4);
+                    const float g = acc[cf][rt][e] * sinv[r];
+                    const float v = a.epi == EPI_ACCUMULATE ? hv[rt][e] + g : g;
+                    if (a.y && n < a.N && row0 + r < a.m) store_through(a.y + (size_t)(row0 + r) * a.y_stride + n, v);
+                    if (a.frag_out) so[r * kOutStride + (2 * nw + cf) * 32 + l32] = v;
+                }
+        }
+    }
+    if (!a.frag_out) return;
+    __syncthreads();
+    // the next GEMM's operand: a wave takes 32 rows x 64 columns at a time
+    const int cols = a.fuse == 1 ? kWideCols / 2 : kWideCols, nck = cols / kChunk;
+    const size_t out_tile = (size_t)(a.n_out / kChunk) * kChunkBytes;
+    for (int it = w; it < kRows / 32 * nck; it += kWideWaves) {
+        const int ch = it % nck, r = (it / nck) * 32 + l32, col = bx * cols + ch * kChunk;
+        if (col >= a.n_out) continue;  // a whole chunk past the outputs
+        float v[32], g[32];
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            const float4 t = *(const float4*)(so + r * kOutStride + ch * kChunk + 32 * hf + 4 * q);
+            const float4 u = a.gain_out ? *(const float4*)(a.gain_out + col + 32 * hf + 4 * q) : make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+            v[4 * q] = t.x, v[4 * q + 1] = t.y, v[4 * q + 2] = t.z, v[4 * q + 3] = t.w;
+            g[4 * q] = u.x, g[4 * q + 1] = u.y, g[4 * q + 2] = u.z, g[4 * q + 3] = u.w;
+        }
+        emit_x_rows(a.frag_out, out_tile, row0 + r, a.m, col / kChunk, v, g, a.order_out, lane);
+    }
+}
+
+// Column tiles [0, a.wide_cols) as workgroups of 128 rows, the others as 64 rows with the chunks in two
+// halves. One dimension, so that the second form's workgroups (half the time each) start as the first
+// form's leave CUs free. Neighbouring workgroups take neighbouring column tiles of the same rows.
+__global__ __launch_bounds__(64 * kWideWaves) void k_gemm_wide(const GemmArgs a) {
+    __shared__ union {
+        WideLds<1> one;
+        WideLds<2> two;
+    } lds;
+    const int id = blockIdx.x, n1 = a.wide_cols, first = n1 * ((a.mpad + 127) / 128);
+    if (id < first) {
+        wide_tile<1>(a, lds.one, id % n1, 0, id / n1);
+    } else {
+        const int n2 = (a.N + kWideCols - 1) / kWideCols - n1, i = id - first;
+        wide_tile<2>(a, lds.two, n1 + i % n2, i / n2 % a.splits, i / n2 / a.splits);
+    }
+}
+
+// How many column tiles run as 128-row workgroups: all, none, or as many as fill whole rounds of the
+// 256 CUs, whichever takes the fewest rounds in all (a 64-row workgroup counts as 0.6 of one: 42
+// against 70 us at K = 2048). Split K and a caller's pass of one row tile take the second form.
+int gemm_wide_cols(int N, int row_tiles, int splits) {
+    const int cols = (N + kWideCols - 1) / kWideCols, mt = (row_tiles + 1) / 2;
+    if (splits > 1) return 0;
+    auto rounds = [](int wgs) { return (wgs + 255) / 256; };
+    int best = 0;
+    float cost = 0.0f;
+    for (int n : {cols, cols * mt / 256 * 256 / mt, 0}) {
+        const float c = (float)rounds(n * mt) + 0.6f * (float)rounds((cols - n) * row_tiles);
+        if (n == cols || c < cost) best = n, cost = c;
+    }
+    return best;
+}
+
+void launch_gemm_wide(GemmArgs a, hipStream_t st) {
+    const int cols = (a.N + kWideCols - 1) / kWideCols;
+    a.wide_cols = gemm_wide_cols(a.N, a.row_tiles, a.splits);
+    const int wgs = a.wide_cols * ((a.mpad + 127) / 128) + (cols - a.wide_cols) * a.splits * (a.mpad / kBM);
+    hipLaunchKernelGGL(k_gemm_wide, dim3(wgs), dim3(64 * kWideWaves), 0, st, a);
+}
+
+}  // namespace qne

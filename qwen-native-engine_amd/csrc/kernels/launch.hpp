@@ -194,6 +194,8 @@ struct GemmArgs {
     uint8_t* frag_out = nullptr;
     const float* gain_out = nullptr;
     int order_out = 0;  // 1: the column order of a q4 GEMM's operand
+    int row_tiles = 1;  // 64-row tiles of the caller's full pass; above 1, q4 runs in gemm_wide.hip
+    int wide_cols = 0;  // set by launch_gemm_wide: column tiles in the 128-row form
     int partials_only = 0;  // write the split partials (even with one split) and launch no reduce:
                             // the kernel that reads the output sums them
 };
@@ -226,6 +228,8 @@ size_t gemm_frag_bytes(int K, int m);
 int gemm_splits(int kind, int N, int K, int group, int row_tiles = 1);
 bool gemm_shape_ok(int kind, int N, int K, int group, int m);
 void launch_gemm(GemmArgs a, hipStream_t st);
+// The GEMM of a pass over a prompt (gemm_wide.hip), called by launch_gemm with the epilogue decided.
+void launch_gemm_wide(GemmArgs a, hipStream_t st);
 // The tile-major copy of q4 (scale, zero) words the row-tiled GEMM reads (GemmArgs::SZT):
 // tile_sz_words(rows, groups) words.
 size_t tile_sz_words(int rows, int ngroups);

@@ -26,6 +26,16 @@ __device__ __forceinline__ void dma4(const void* src, void* dst) {
     asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %1, off\n\ts_mov_b32 m0, %0"
                  : "=&s"(saved) : "v"(src), "s"(lds) : "memory");
 }
+// The LDS address of a pointer into LDS (wave-uniform), and dma16 from a wave-uniform base plus a
+// 32-bit byte offset per lane to such an address.
+__device__ __forceinline__ uint32_t lds_address(const void* p) {
+    return __builtin_amdgcn_readfirstlane((uint32_t)(size_t)(lds_ptr_t)p);
+}
+__device__ __forceinline__ void dma16_at(const void* base, uint32_t offset, uint32_t lds) {
+    uint32_t saved;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
+                 : "=&s"(saved) : "v"(offset), "s"(base), "s"(lds) : "memory");
+}
 // Until at most N of this wave's vector-memory operations are outstanding (they complete in issue
 // order); the memory clobber keeps the LDS reads of the landed data after it.
 template <int N>

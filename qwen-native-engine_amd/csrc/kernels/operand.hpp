@@ -36,6 +36,7 @@ __device__ __forceinline__ int frag_offset(int s, int mt, int lane) { return ((s
 // the previous one.
 __device__ __forceinline__ void emit_x(uint8_t* __restrict__ frag, size_t tile_bytes, int r, int c, float v, float g,
                                        int q4order, int lane) {
+#pragma clang fp contract(off)  // the sums' rounding is the same wherever an operand is staged
     const float xg = v * g;
     const float hi = (float)(_Float16)xg;
     const float lo = (float)(_Float16)(xg - hi);
@@ -51,6 +52,54 @@ __device__ __forceinline__ void emit_x(uint8_t* __restrict__ frag, size_t tile_b
         float* sums = (float*)tile;
         sums[kXsumOff / 4 + rr] = xs;
         sums[kSsOff / 4 + rr] = ss;
+    }
+}
+
+// The same for a wave that holds 32 rows of one chunk: lane 32 hf + row has the chunk's columns
+// 32 hf + 8 s + i (s, i: v[8 s + i], times g[8 s + i]) of row r = 32 k + row, so each half's eight
+// stores are whole contiguous KiB (emit_x: 2 bytes a lane). The sums are added in emit_x's order
+// (a balanced tree over the columns), so the operand's bits are the same. Rows >= m are not written.
+__device__ __forceinline__ void emit_x_rows(uint8_t* __restrict__ frag, size_t tile_bytes, int r, int m, int chunk,
+                                            const float (&v)[32], const float (&g)[32], int q4order, int lane) {
+#pragma clang fp contract(off)
+    uint8_t* tile = frag + (size_t)(r / kBM) * tile_bytes + (size_t)chunk * kChunkBytes;
+    const int rr = r & (kBM - 1);
+    float xs[4], ss[4];
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        uint16_t hi[8], lo[8];
+        float xt[8], st[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const float xg = v[8 * s + i] * g[8 * s + i];
+            const _Float16 h = (_Float16)xg, l = (_Float16)(xg - (float)h);
+            hi[i] = __builtin_bit_cast(uint16_t, h);
+            lo[i] = __builtin_bit_cast(uint16_t, l);
+            xt[i] = (float)h + (float)l;
+            st[i] = v[8 * s + i] * v[8 * s + i];
+        }
+        xs[s] = ((xt[0] + xt[1]) + (xt[2] + xt[3])) + ((xt[4] + xt[5]) + (xt[6] + xt[7]));
+        ss[s] = ((st[0] + st[1]) + (st[2] + st[3])) + ((st[4] + st[5]) + (st[6] + st[7]));
+        uint32_t hw[4], lw[4];
+#pragma unroll
+        for (int p = 0; p < 4; p++) {  // word p: slots 2 p, 2 p + 1 (q4 order: columns p, p + 4)
+            const int a = 2 * p, b = 2 * p + 1;
+            hw[p] = q4order ? hi[p] | (uint32_t)hi[p + 4] << 16 : hi[a] | (uint32_t)hi[b] << 16;
+            lw[p] = q4order ? lo[p] | (uint32_t)lo[p + 4] << 16 : lo[a] | (uint32_t)lo[b] << 16;
+        }
+        if (r < m) {
+            uint8_t* dst = tile + frag_offset(s, rr >> 5, lane);
+            *(uint4*)dst = make_uint4(hw[0], hw[1], hw[2], hw[3]);
+            *(uint4*)(dst + kFragBytes) = make_uint4(lw[0], lw[1], lw[2], lw[3]);
+        }
+    }
+    float xt = (xs[0] + xs[1]) + (xs[2] + xs[3]), st = (ss[0] + ss[1]) + (ss[2] + ss[3]);
+    xt += lane_xor32(xt, lane);
+    st += lane_xor32(st, lane);
+    if (r < m && lane < 32) {
+        float* sums = (float*)tile;
+        sums[kXsumOff / 4 + rr] = xt;
+        sums[kSsOff / 4 + rr] = st;
     }
 }
 

@@ -85,6 +85,22 @@ def test_gemm_full_pass_of_rows(M):
     assert rel_err(got, want) < 2e-5
 
 
+@pytest.mark.parametrize("rows,k,group,M,epi", [
+    (256, 64, 64, 257, Q.EPI_STORE),            # one chunk: the odd half of the 64-row form has none
+    (300, 320, 64, 300, Q.EPI_ACCUMULATE),      # five chunks, split; a ragged column tile, waves past N
+    (520, 128, 128, 333, Q.EPI_STORE),          # two chunks of one scale group, one split
+    (512, 192, 64, 321, Q.EPI_SWIGLU),          # SwiGLU by the GEMM, an odd last row tile
+    (360, 1024, 128, 450, Q.EPI_SWIGLU),        # SwiGLU by the reduce (180 outputs)
+    (4128, 192, 64, 1990, Q.EPI_ACCUMULATE),    # 16 column tiles as 128 rows, the ragged 17th as 64
+    (4096, 1088, 64, 2048, Q.EPI_SWIGLU),       # 17 chunks: a second batch of the zero points' sums
+])
+def test_gemm_wide_forms(rows, k, group, M, epi):
+    """Calls above 256 rows: both workgroup forms, at the edges of tiles, chunks and halves. The bar is
+    the GEMM's; the sums here are closer (one rounding per chunk, exact zero points)."""
+    got, want = run_gemm(Q.MAT_Q4, group, rows, k, M, epi, True, seed=rows + k + M)
+    assert rel_err(got, want) < 2e-5
+
+
 @pytest.mark.parametrize("kind,group", [(Q.MAT_Q4, 64), (Q.MAT_F16, 0)])
 def test_gemm_one_split_direct_epilogue(kind, group):
     """More than 512 tiles of 128 rows: one split, the GEMM applies 1 / rms and the epilogue itself
