@@ -1,5 +1,6 @@
 // extern "C" boundary (include/qne.h): every call catches, maps the error to a return code and
 // keeps the message for qne_last_error().
+#include <algorithm>
 #include <hip/hip_runtime.h>
 
 #include <cstring>
@@ -380,7 +381,12 @@ int qne_gemm(int kind, const void* w, const void* sz, int rows, int k, int group
         // up to 256 rows share one split count and form, so a row's sums do not depend on the call;
         // longer calls would write a partial of every row per split and run as a prompt's pass
         if (m > 256 && kind == QNE_MAT_Q4) a.row_tiles = (m + 63) / 64;
+        // (and at least 8 chunks a split: 400 x 100 x 2048 with two took 23 us)
         a.splits = qne::gemm_splits(kind, rows, k, a.group, a.row_tiles);
+        if (a.row_tiles > 1) {
+            const int nch = k / 64, most = std::max(1, std::min(a.splits, nch / 8)), per = (nch + most - 1) / most;
+            a.splits = (nch + per - 1) / per;  // no empty split
+        }
         a.epi = epilogue;
         a.y = y;
         a.y_stride = y_stride;

@@ -54,6 +54,28 @@ __global__ __launch_bounds__(256) void k_stage_x(const float* __restrict__ x, in
     emit_x(frag, (size_t)(K / kChunk) * kChunkBytes, r, c, v, gain ? gain[c] : 1.0f, q4order, threadIdx.x & 63);
 }
 
+typedef float float4a_t __attribute__((ext_vector_type(4), aligned(4)));  // the caller's rows: any float
+
+// The same for many rows, grid (ceil(K / 256), rows / 32): a wave takes 32 rows of a chunk, half a row
+// (128 contiguous bytes) a lane, and stores 16 bytes a lane instead of 2. Memory-bound: 2048 x 2048
+// 15 -> 9.9 us, 2048 x 6144 32 -> 22 us; with few rows too few waves are in flight (64 x 2048 4 -> 6 us).
+__global__ __launch_bounds__(256) void k_stage_x_rows(const float* __restrict__ x, int x_stride, int m, int K,
+                                                      const float* __restrict__ gain, int q4order, uint8_t* __restrict__ frag) {
+    const int lane = threadIdx.x & 63, chunk = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (chunk * kChunk >= K) return;  // whole wave
+    const int r = blockIdx.y * 32 + (lane & 31), c = chunk * kChunk + 32 * (lane >> 5);
+    float v[32], g[32];
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+        float4a_t t = {0.0f, 0.0f, 0.0f, 0.0f}, u = {1.0f, 1.0f, 1.0f, 1.0f};
+        if (r < m) t = *(const float4a_t*)(x + (size_t)r * x_stride + c + 4 * q);
+        if (gain) u = *(const float4a_t*)(gain + c + 4 * q);
+        v[4 * q] = t.x, v[4 * q + 1] = t.y, v[4 * q + 2] = t.z, v[4 * q + 3] = t.w;
+        g[4 * q] = u.x, g[4 * q + 1] = u.y, g[4 * q + 2] = u.z, g[4 * q + 3] = u.w;
+    }
+    emit_x_rows(frag, (size_t)(K / kChunk) * kChunkBytes, r, r + 1, chunk, v, g, q4order, lane);
+}
+
 // Until at most n of the wave's vector-memory operations are outstanding (n wave-uniform; counts
 // past 31 wait for 31, which is only stricter).
 __device__ __forceinline__ void wait_vm_upto(int n) {
@@ -542,7 +564,11 @@ size_t gemm_frag_bytes(int K, int m) { return (size_t)((m + kBM - 1) / kBM) * (K
 void launch_stage_x(const float* x, int x_stride, int m, int K, const float* gain, int q4order, uint8_t* frag,
                     hipStream_t st) {
     const int mpad = (m + kBM - 1) / kBM * kBM;
-    hipLaunchKernelGGL(k_stage_x, dim3((K + 255) / 256, mpad), dim3(256), 0, st, x, x_stride, m, K, gain, q4order, frag);
+    const int wgs = (K + 255) / 256 * (mpad / 32);
+    if (wgs >= 256)
+        hipLaunchKernelGGL(k_stage_x_rows, dim3((K + 255) / 256, mpad / 32), dim3(256), 0, st, x, x_stride, m, K, gain, q4order, frag);
+    else
+        hipLaunchKernelGGL(k_stage_x, dim3((K + 255) / 256, mpad), dim3(256), 0, st, x, x_stride, m, K, gain, q4order, frag);
 }
 
 // The tile-major copy of a q4 matrix's (scale, zero) words: szt[(t G + g) 32 + r] = sz[(32 t + r) G + g]
@@ -581,7 +607,8 @@ void launch_gemm(GemmArgs a, hipStream_t st) {
     const bool dma_waves = a.mpad == kBM && !wide;
     // One split over several row tiles: the GEMM applies the SwiGLU, or the store / residual add,
     // and stages the output itself, with no partials and no reduce pass
-    const bool one = a.fuse == 0 && a.kind == KIND_Q4 && !dma_waves && a.splits == 1 && !a.partials_only;
+    const bool few = wide && gemm_is_short(a);  // writes partials
+    const bool one = a.fuse == 0 && a.kind == KIND_Q4 && !dma_waves && a.splits == 1 && !a.partials_only && !few;
     a.fuse = 0;
     if (one && a.epi == EPI_SWIGLU && a.N == 2 * a.n_out && a.n_out % (32 * waves / 2) == 0 && a.K <= 64 * kChunk &&
         (a.y || a.frag_out))
@@ -590,7 +617,7 @@ void launch_gemm(GemmArgs a, hipStream_t st) {
     else if (one && wide && a.epi != EPI_SWIGLU && a.frag_out && a.n_out == a.N && a.N % kChunk == 0 &&
              (a.epi == EPI_STORE || a.y) && (!a.norm || a.K <= 64 * kChunk))
         a.fuse = 2;
-    a.direct = a.splits == 1 && a.epi != EPI_SWIGLU && !a.frag_out && !a.partials_only;
+    a.direct = a.splits == 1 && a.epi != EPI_SWIGLU && !a.frag_out && !a.partials_only && !few;
     if (wide) {
         launch_gemm_wide(a, st);
     } else if (a.kind == KIND_Q4) {

@@ -422,6 +422,150 @@ __global__ __launch_bounds__(64 * kWideWaves) void k_gemm_wide(const GemmArgs a)
     }
 }
 
+// The same sums for a call of few rows, where the workgroups above would leave most CUs idle (64 rows,
+// N = 2048: 8 of them, 43 us). A workgroup takes 32 rows x 32 CT columns, and its 8 waves take 8
+// chunks at once: the products of a chunk do not depend on the other chunks', only the fma that scales
+// them into the accumulator does. So each wave forms its chunk's products, from x and W straight out of
+// L2 (nothing is shared between the waves), and leaves them in LDS, where wave w adds the 8 chunks'
+// products of its 2 CT of the tile's accumulator registers in chunk order: the sums are bit for bit
+// those of wide_tile. Every workgroup streams its rows of x whole, which bounds it (64 bytes a clock and
+// CU; 264 KB at K = 2048). Writes split partials; the reduce applies the epilogue.
+// Grid (ceil(N / (32 CT)), splits, ceil(m / 32)).
+template <int CT>
+__global__ __launch_bounds__(64 * kWideWaves) void k_gemm_short(const GemmArgs a) {
+    constexpr int OWN = 2 * CT;                     // accumulator registers of a wave
+    __shared__ float prod[kWideWaves][16 * CT][64];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int hf = lane >> 5, l32 = lane & 31;
+    const int nchunks = a.K / kChunk, cpg = a.group / kChunk, ngroups = nchunks / cpg;
+    const int c0 = blockIdx.y * a.cps, c1 = min(nchunks, c0 + a.cps), nch = c1 - c0;
+    const int row0 = blockIdx.z * 32, col0 = blockIdx.x * 32 * CT;
+    const bool two = col0 / kWideCols >= a.wide_cols;  // even and odd chunks apart (the 64-row form)
+    const uint8_t* xtile = a.frag + (size_t)(row0 / kBM) * nchunks * kChunkBytes;
+    const int rt = (row0 / 32) & 1;                 // which half of the 64-row tile
+    const uint32_t* szt[CT];
+    const uint8_t* wrow[CT];
+#pragma unroll
+    for (int t = 0; t < CT; t++) {
+        const int r = min(col0 + 32 * t, a.N - 1);
+        szt[t] = a.SZT + (size_t)(r >> 5) * ngroups * 32 + l32;
+        wrow[t] = (const uint8_t*)a.W + (size_t)min(col0 + 32 * t + l32, a.N - 1) * (a.K / 2) + 16 * hf;
+    }
+    const uint64_t inv_cpg = (uint64_t)(0xFFFFFFFFu / (unsigned)cpg) + 1;  // ceil(2^32 / cpg): c / cpg with no branch
+    auto group = [&](int c) -> int { return (int)(((uint64_t)(unsigned)c * inv_cpg) >> 32); };
+    const int own_t = w * OWN / 16, own_e = w * OWN % 16;  // this wave's column tile and registers
+
+    struct Operands {
+        half8_t h[4], l[4];
+        uint4 w[CT];
+        uint32_t sz[kWideWaves];
+    } ops[2];  // of two rounds: one computed, the next one's loads in flight
+    auto load = [&](Operands& o, int r) {  // round r: this wave's chunk, and the scales of all of them
+        const int c = c0 + min(8 * r + w, nch - 1);
+        const uint8_t* xs = xtile + (size_t)c * kChunkBytes;
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            o.h[s] = *(const half8_t*)(xs + frag_offset(s, rt, lane));
+            o.l[s] = *(const half8_t*)(xs + kFragBytes + frag_offset(s, rt, lane));
+        }
+#pragma unroll
+        for (int t = 0; t < CT; t++) o.w[t] = *(const uint4*)(wrow[t] + (size_t)c * 32);
+        const uint32_t* sp = CT == 1 || own_t == 0 ? szt[0] : szt[CT - 1];
+#pragma unroll
+        for (int k = 0; k < kWideWaves; k++) o.sz[k] = sp[(size_t)group(c0 + min(8 * r + k, nch - 1)) * 32];
+    };
+    load(ops[0], 0);
+
+    // the accumulators' first values, as in wide_tile: wave (parity, column tile)
+    if (w < (two ? 2 : 1) * CT) {
+        const int t = w % CT, step = two ? 2 : 1, cfirst = c0 + w / CT, nmine = (c1 - cfirst + step - 1) / step;
+        const float* xsum = (const float*)(xtile + kXsumOff) + 32 * rt + l32;
+        float16_t z = {};
+        for (int b = 0; b < nmine; b += 16) {
+            Bf3 xa, wb;
+            float xv[8];
+            uint32_t sv[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const int c = cfirst + step * min(b + 8 * hf + i, nmine - 1);
+                xv[i] = xsum[(size_t)c * (kChunkBytes / 4)];
+                sv[i] = (CT == 1 || t == 0 ? szt[0] : szt[CT - 1])[(size_t)group(c) * 32];
+            }
+#pragma unroll
+            for (int i = 0; i < 8; i++) asm volatile("" : "+v"(xv[i]), "+v"(sv[i]));  // keeps the loads together
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const bool live = b + 8 * hf + i < nmine;
+                xa.set(i, live ? xv[i] : 0.0f);
+                wb.set(i, live ? lo_h(sv[i]) * (8.0f - hi_h(sv[i])) : 0.0f);
+            }
+#pragma unroll
+            for (int p = 2; p >= 0; p--)
+#pragma unroll
+                for (int q = 0; q <= p; q++) z = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa.t[q], wb.t[p - q], z, 0, 0, 0);
+        }
+#pragma unroll
+        for (int e = 0; e < 16; e++) prod[w / CT][16 * t + e][lane] = z[e];
+    }
+    __syncthreads();
+    float acc[2][OWN];
+#pragma unroll
+    for (int i = 0; i < OWN; i++) {
+        acc[0][i] = prod[0][w * OWN + i][lane];
+        acc[1][i] = two ? prod[1][w * OWN + i][lane] : 0.0f;
+    }
+    const int rounds = (nch + kWideWaves - 1) / kWideWaves;
+    auto round = [&](const Operands& cur, int r) {
+        float16_t grp[CT] = {};
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            half8_t b[CT];
+#pragma unroll
+            for (int t = 0; t < CT; t++) b[t] = nibbles8_signed(s == 0 ? cur.w[t].x : s == 1 ? cur.w[t].y : s == 2 ? cur.w[t].z : cur.w[t].w);
+#pragma unroll
+            for (int t = 0; t < CT; t++) grp[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(cur.h[s], b[t], grp[t], 0, 0, 0);
+#pragma unroll
+            for (int t = 0; t < CT; t++) grp[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(cur.l[s], b[t], grp[t], 0, 0, 0);
+        }
+        __syncthreads();  // the previous round's products are used
+#pragma unroll
+        for (int t = 0; t < CT; t++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) prod[w][16 * t + e][lane] = grp[t][e];
+        __syncthreads();
+        float p[kWideWaves][OWN];
+#pragma unroll
+        for (int k = 0; k < kWideWaves; k++)
+#pragma unroll
+            for (int i = 0; i < OWN; i++) p[k][i] = prod[k][w * OWN + i][lane];
+        const int live = nch - kWideWaves * r;  // chunks past the split leave the sums as they are
+#pragma unroll
+        for (int k = 0; k < kWideWaves; k++) {
+            const float sc = lo_h(cur.sz[k]);
+#pragma unroll
+            for (int i = 0; i < OWN; i++) {
+                float& d = two ? acc[k & 1][i] : acc[0][i];
+                const float v = fmaf(sc, p[k][i], d);
+                d = k < live ? v : d;
+            }
+        }
+    };
+    for (int r = 0; r < rounds; r += 2) {
+        load(ops[1], r + 1);
+        round(ops[0], r);
+        if (r + 1 >= rounds) break;
+        load(ops[0], r + 2);
+        round(ops[1], r + 1);
+    }
+    const int n = col0 + 32 * own_t + l32;
+    if (n >= a.N) return;
+#pragma unroll
+    for (int i = 0; i < OWN; i++) {
+        const int e = own_e + i, r = row0 + 8 * (e / 4) + 4 * hf + (e % 4);
+        store_through(a.part + ((size_t)blockIdx.y * a.mpad + r) * a.N + n, two ? acc[0][i] + acc[1][i] : acc[0][i]);
+    }
+}
+
 // How many column tiles run as 128-row workgroups: all, none, or as many as fill whole rounds of the
 // 256 CUs, whichever takes the fewest rounds in all (a 64-row workgroup counts as 0.6 of one: 42
 // against 70 us at K = 2048). Split K and a caller's pass of one row tile take the second form.
@@ -438,9 +582,26 @@ int gemm_wide_cols(int N, int row_tiles, int splits) {
     return best;
 }
 
+// Where the short form (with its reduce) beats wide_tile, both measured on the 2B model's matrices, mean
+// over the layers, us, short / wide: N = 2048, 64 rows 24 / 59, 256 rows (256 workgroups) 33 / 59, 512
+// rows (512) 53 / 60; N = 8224, 64 rows 32 / 57, 128 rows (516) 49 / 57, 256 rows (1032) 81 / 58; N =
+// 12288, 128 rows (768) 51 / 57, 256 rows (1536) 93 / 60.
+bool gemm_is_short(const GemmArgs& a) {
+    const int wgs = (a.N + 63) / 64 * ((a.m + 31) / 32) * a.splits;
+    return wgs <= (a.m <= 128 ? 768 : 512);
+}
+
 void launch_gemm_wide(GemmArgs a, hipStream_t st) {
     const int cols = (a.N + kWideCols - 1) / kWideCols;
     a.wide_cols = gemm_wide_cols(a.N, a.row_tiles, a.splits);
+    if (!a.fuse && !a.direct && gemm_is_short(a)) {
+        const int tiles = (a.m + 31) / 32;
+        if ((a.N + 63) / 64 * tiles * a.splits < 256)
+            hipLaunchKernelGGL(k_gemm_short<1>, dim3((a.N + 31) / 32, a.splits, tiles), dim3(64 * kWideWaves), 0, st, a);
+        else
+            hipLaunchKernelGGL(k_gemm_short<2>, dim3((a.N + 63) / 64, a.splits, tiles), dim3(64 * kWideWaves), 0, st, a);
+        return;
+    }
     const int wgs = a.wide_cols * ((a.mpad + 127) / 128) + (cols - a.wide_cols) * a.splits * (a.mpad / kBM);
     hipLaunchKernelGGL(k_gemm_wide, dim3(wgs), dim3(64 * kWideWaves), 0, st, a);
 }

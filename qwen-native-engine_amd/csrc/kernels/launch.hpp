@@ -229,6 +229,8 @@ int gemm_splits(int kind, int N, int K, int group, int row_tiles = 1);
 bool gemm_shape_ok(int kind, int N, int K, int group, int m);
 void launch_gemm(GemmArgs a, hipStream_t st);
 // The GEMM of a pass over a prompt (gemm_wide.hip), called by launch_gemm with the epilogue decided.
+// A call of few rows (gemm_is_short) writes split partials only.
+bool gemm_is_short(const GemmArgs& a);
 void launch_gemm_wide(GemmArgs a, hipStream_t st);
 // The tile-major copy of q4 (scale, zero) words the row-tiled GEMM reads (GemmArgs::SZT):
 // tile_sz_words(rows, groups) words.
