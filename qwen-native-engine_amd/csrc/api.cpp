@@ -398,11 +398,7 @@ int qne_gemm(int kind, const void* w, const void* sz, int rows, int k, int group
         a.part = ws;
         a.frag = (uint8_t*)(ws + part);
         hipStream_t st = (hipStream_t)stream;
-        if (szt) {  // the GEMM reads the words tile-major
-            uint32_t* d = (uint32_t*)(a.frag + frag);
-            qne::launch_tile_sz((const uint32_t*)sz, rows, k / a.group, d, st);
-            a.SZT = d;
-        }
+        if (szt) a.szt_build = (uint32_t*)(a.frag + frag);
         qne::launch_gemm(a, st);
         check_launch();
         if (!stream) qne::hip_check(hipStreamSynchronize(st), "gemm");

@@ -42,38 +42,71 @@ __device__ __forceinline__ uint32_t pack_h2(float a, float b) {
 
 }  // namespace
 
-// Grid (ceil(K / 256), rows rounded up to 64): the x operand of a GEMM from f32 rows
-// (x + r * x_stride; rows >= m are zero), times `gain` when set; the row's RMSNorm factor is applied
-// by the GEMM's epilogue.
-__global__ __launch_bounds__(256) void k_stage_x(const float* __restrict__ x, int x_stride, int m, int K,
-                                                 const float* __restrict__ gain, int q4order, uint8_t* __restrict__ frag) {
-    const int c = blockIdx.x * 256 + threadIdx.x, r = blockIdx.y;
-    if (blockIdx.x * 256 >= K) return;  // whole workgroup; K is a multiple of 64, so waves are whole chunks
-    if ((threadIdx.x & ~63) + blockIdx.x * 256 >= K) return;  // whole wave
-    const float v = r < m ? x[(size_t)r * x_stride + c] : 0.0f;
-    emit_x(frag, (size_t)(K / kChunk) * kChunkBytes, r, c, v, gain ? gain[c] : 1.0f, q4order, threadIdx.x & 63);
+// The x operand of a GEMM from f32 rows (x + r * x_stride; rows >= m are zero), times `gain` when set;
+// the row's RMSNorm factor is applied by the GEMM's epilogue.
+struct StageArgs {
+    const float* x;
+    int x_stride, m, K;
+    const float* gain;
+    int q4order;
+    uint8_t* frag;
+    // with sz, also the tile-major copy of a q4 matrix's (scale, zero) words: szt[(t G + g) 32 + r] =
+    // sz[(32 t + r) G + g] (zero for rows past the matrix)
+    const uint32_t* sz;
+    int rows, ngroups;
+    uint32_t* szt;
+};
+
+// One value a lane: workgroup (bx, r) stages columns 256 bx.. of row r.
+__device__ __forceinline__ void stage_columns(const StageArgs& a, int bx, int r) {
+    const int c = bx * 256 + threadIdx.x;
+    if ((int)(threadIdx.x & ~63) + bx * 256 >= a.K) return;  // whole wave; K is a multiple of 64
+    const float v = r < a.m ? a.x[(size_t)r * a.x_stride + c] : 0.0f;
+    emit_x(a.frag, (size_t)(a.K / kChunk) * kChunkBytes, r, c, v, a.gain ? a.gain[c] : 1.0f, a.q4order, threadIdx.x & 63);
 }
 
 typedef float float4a_t __attribute__((ext_vector_type(4), aligned(4)));  // the caller's rows: any float
 
-// The same for many rows, grid (ceil(K / 256), rows / 32): a wave takes 32 rows of a chunk, half a row
-// (128 contiguous bytes) a lane, and stores 16 bytes a lane instead of 2. Memory-bound: 2048 x 2048
-// 15 -> 9.9 us, 2048 x 6144 32 -> 22 us; with few rows too few waves are in flight (64 x 2048 4 -> 6 us).
-__global__ __launch_bounds__(256) void k_stage_x_rows(const float* __restrict__ x, int x_stride, int m, int K,
-                                                      const float* __restrict__ gain, int q4order, uint8_t* __restrict__ frag) {
-    const int lane = threadIdx.x & 63, chunk = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (chunk * kChunk >= K) return;  // whole wave
-    const int r = blockIdx.y * 32 + (lane & 31), c = chunk * kChunk + 32 * (lane >> 5);
+// 32 rows of a chunk a wave, half a row (128 contiguous bytes) a lane, stored 16 bytes a lane instead of
+// 2: workgroup (bx, by) stages columns 256 bx.. of rows 32 by... Memory-bound: 2048 x 2048 15 -> 9.9 us,
+// 2048 x 6144 32 -> 22 us; with few rows too few waves are in flight (64 x 2048 4 -> 6 us).
+__device__ __forceinline__ void stage_rows(const StageArgs& a, int bx, int by) {
+    const int lane = threadIdx.x & 63, chunk = bx * 4 + (threadIdx.x >> 6);
+    if (chunk * kChunk >= a.K) return;  // whole wave
+    const int r = by * 32 + (lane & 31), c = chunk * kChunk + 32 * (lane >> 5);
     float v[32], g[32];
 #pragma unroll
     for (int q = 0; q < 8; q++) {
         float4a_t t = {0.0f, 0.0f, 0.0f, 0.0f}, u = {1.0f, 1.0f, 1.0f, 1.0f};
-        if (r < m) t = *(const float4a_t*)(x + (size_t)r * x_stride + c + 4 * q);
-        if (gain) u = *(const float4a_t*)(gain + c + 4 * q);
+        if (r < a.m) t = *(const float4a_t*)(a.x + (size_t)r * a.x_stride + c + 4 * q);
+        if (a.gain) u = *(const float4a_t*)(a.gain + c + 4 * q);
         v[4 * q] = t.x, v[4 * q + 1] = t.y, v[4 * q + 2] = t.z, v[4 * q + 3] = t.w;
         g[4 * q] = u.x, g[4 * q + 1] = u.y, g[4 * q + 2] = u.z, g[4 * q + 3] = u.w;
     }
-    emit_x_rows(frag, (size_t)(K / kChunk) * kChunkBytes, r, r + 1, chunk, v, g, q4order, lane);
+    emit_x_rows(a.frag, (size_t)(a.K / kChunk) * kChunkBytes, r, r + 1, chunk, v, g, a.q4order, lane);
+}
+
+// Tile t's words of groups 64 piece..: rows read whole, turned in LDS, written as whole lines.
+__device__ __forceinline__ void tile_words(const StageArgs& a, uint32_t (*words)[65], int t, int piece) {
+    const int g0 = 64 * piece, ng = min(64, a.ngroups - g0);
+    for (int i = threadIdx.x; i < 32 * 64; i += 256) {
+        const int r = i / 64, g = i % 64;
+        if (g < ng) words[r][g] = 32 * t + r < a.rows ? a.sz[(size_t)(32 * t + r) * a.ngroups + g0 + g] : 0u;
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < 32 * ng; i += 256) a.szt[((size_t)t * a.ngroups + g0) * 32 + i] = words[i % 32][i / 32];
+}
+
+// What a GEMM call on the caller's rows needs first, in one launch: the words' tiles (ceil(rows / 32) x
+// ceil(G / 64) workgroups, none without sz), then x. Two launches, the words 4 bytes a lane from 32 rows:
+// 4 us more on a call of 20 to 50.
+template <bool ROWS>
+__global__ __launch_bounds__(256) void k_stage(const StageArgs a, int word_tiles, int pieces) {
+    __shared__ uint32_t words[32][65];
+    const int wgs = word_tiles * pieces, id = (int)blockIdx.x - wgs, nx = (a.K + 255) / 256;
+    if (id < 0) tile_words(a, words, blockIdx.x / pieces, blockIdx.x % pieces);
+    else if (ROWS) stage_rows(a, id % nx, id / nx);
+    else stage_columns(a, id % nx, id / nx);
 }
 
 // Until at most n of the wave's vector-memory operations are outstanding (n wave-uniform; counts
@@ -561,40 +594,32 @@ bool gemm_shape_ok(int kind, int N, int K, int group, int m) {
 
 size_t gemm_frag_bytes(int K, int m) { return (size_t)((m + kBM - 1) / kBM) * (K / kChunk) * kChunkBytes; }
 
-void launch_stage_x(const float* x, int x_stride, int m, int K, const float* gain, int q4order, uint8_t* frag,
-                    hipStream_t st) {
-    const int mpad = (m + kBM - 1) / kBM * kBM;
-    const int wgs = (K + 255) / 256 * (mpad / 32);
-    if (wgs >= 256)
-        hipLaunchKernelGGL(k_stage_x_rows, dim3((K + 255) / 256, mpad / 32), dim3(256), 0, st, x, x_stride, m, K, gain, q4order, frag);
-    else
-        hipLaunchKernelGGL(k_stage_x, dim3((K + 255) / 256, mpad), dim3(256), 0, st, x, x_stride, m, K, gain, q4order, frag);
-}
-
-// The tile-major copy of a q4 matrix's (scale, zero) words: szt[(t G + g) 32 + r] = sz[(32 t + r) G + g]
-// (zero for rows past the matrix). Grid (ceil(rows / 32) G / 8), 256 threads.
-__global__ __launch_bounds__(256) void k_tile_sz(const uint32_t* __restrict__ sz, int rows, int ngroups,
-                                                 uint32_t* __restrict__ szt) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, tiles = ((size_t)rows + 31) / 32;
-    if (i >= tiles * ngroups * 32) return;
-    const size_t r = (i / ((size_t)ngroups * 32)) * 32 + i % 32, g = (i / 32) % ngroups;
-    szt[i] = r < (size_t)rows ? sz[r * ngroups + g] : 0u;
-}
-
 size_t tile_sz_words(int rows, int ngroups) { return ((size_t)rows + 31) / 32 * ngroups * 32; }
 
-void launch_tile_sz(const uint32_t* sz, int rows, int ngroups, uint32_t* szt, hipStream_t st) {
-    const size_t n = tile_sz_words(rows, ngroups);
-    hipLaunchKernelGGL(k_tile_sz, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, sz, rows, ngroups, szt);
+static void launch_stage(const GemmArgs& a, hipStream_t st) {
+    StageArgs s{a.x, a.x_stride, a.m, a.K, a.gain, a.kind == KIND_Q4 ? 1 : 0, a.frag, nullptr, 0, 0, nullptr};
+    int tiles = 0, pieces = 0;
+    if (a.szt_build) {
+        s.sz = a.SZ;
+        s.rows = a.N;
+        s.ngroups = a.K / a.group;
+        s.szt = a.szt_build;
+        tiles = (a.N + 31) / 32;
+        pieces = (s.ngroups + 63) / 64;
+    }
+    const int nx = (a.K + 255) / 256, wgs = nx * (a.mpad / 32);
+    if (wgs >= 256) hipLaunchKernelGGL(k_stage<true>, dim3(tiles * pieces + wgs), dim3(256), 0, st, s, tiles, pieces);
+    else hipLaunchKernelGGL(k_stage<false>, dim3(tiles * pieces + nx * a.mpad), dim3(256), 0, st, s, tiles, pieces);
 }
 
 void launch_gemm(GemmArgs a, hipStream_t st) {
+    if (a.szt_build) a.SZT = a.szt_build;
     if (a.kind == KIND_Q4 && !a.SZT) throw Error(QNE_EINVAL, "q4 GEMM needs the tile-major scale/zero words");
     const int nch = a.K / kChunk;
     a.cps = (nch + a.splits - 1) / a.splits;
     a.mpad = (a.m + kBM - 1) / kBM * kBM;
     if (a.x) {  // stage the x operand here (RMSNorm gain folded in, 1 / rms deferred to the epilogue)
-        launch_stage_x(a.x, a.x_stride, a.m, a.K, a.gain, a.kind == KIND_Q4 ? 1 : 0, a.frag, st);
+        launch_stage(a, st);
         a.norm = a.gain ? 1 : 0;
     }
     const bool wide = a.kind == KIND_Q4 && a.row_tiles > 1;

@@ -179,6 +179,7 @@ struct GemmArgs {
     const void* W = nullptr;
     const uint32_t* SZ = nullptr;
     const uint32_t* SZT = nullptr;  // q4: SZ tile-major ([row / 32][group][row % 32]), what k_gemm reads
+    uint32_t* szt_build = nullptr;  // with x set: where launch_gemm makes SZT from SZ first
     int N = 0, K = 0, group = 64;
     int splits = 1;
     int cps = 0;     // set by launch_gemm: chunks per split
@@ -235,10 +236,6 @@ void launch_gemm_wide(GemmArgs a, hipStream_t st);
 // The tile-major copy of q4 (scale, zero) words the row-tiled GEMM reads (GemmArgs::SZT):
 // tile_sz_words(rows, groups) words.
 size_t tile_sz_words(int rows, int ngroups);
-void launch_tile_sz(const uint32_t* sz, int rows, int ngroups, uint32_t* szt, hipStream_t st);
-// The x operand of a GEMM from f32 rows (rows >= m zero), times gain when set.
-void launch_stage_x(const float* x, int x_stride, int m, int K, const float* gain, int q4order, uint8_t* frag,
-                    hipStream_t st);
 // h[r] = embedding row tokens[r], r < m; with frag, h * gain is also staged as a GEMM's x operand.
 // With order, order[0..m) = the rows 0..m-1 by decreasing pos (ties: lower row first), the order
 // the attention partials run them in.
