@@ -2,6 +2,8 @@
 // count. Weights are the Model's; every row has its own recurrent state and paged KV cache.
 #include "batch.hpp"
 
+#include <omp.h>
+
 #include <algorithm>
 #include <cstring>
 #include <random>
@@ -167,6 +169,8 @@ BatchDecoder::BatchDecoder(Model& m, int max_rows, int max_context) : m_(m), max
         QNE_HIP(hipMemset(tokens_, 0, kRowsMax * 4));
         QNE_HIP(hipMemset(pos_, 0, kRowsMax * 4));
         QNE_HIP(hipHostMalloc((void**)&host_u32_, 2 * kRowsMax * 4, hipHostMallocDefault));
+        QNE_HIP(hipHostMalloc((void**)&host_read_, kReadSlots * kReadSlot, hipHostMallocDefault));
+        for (hipEvent_t& e : read_ev_) QNE_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     } catch (...) {
         release();
         throw;
@@ -184,6 +188,12 @@ void BatchDecoder::release() {
     allocations_.clear();
     if (host_u32_) (void)hipHostFree(host_u32_);
     host_u32_ = nullptr;
+    if (host_read_) (void)hipHostFree(host_read_);
+    host_read_ = nullptr;
+    for (hipEvent_t& e : read_ev_) {
+        if (e) (void)hipEventDestroy(e);
+        e = nullptr;
+    }
     if (ev0_) (void)hipEventDestroy(ev0_);
     if (ev1_) (void)hipEventDestroy(ev1_);
     ev0_ = ev1_ = nullptr;
@@ -397,6 +407,44 @@ void BatchDecoder::row_state(int n, uint32_t* tokens, uint32_t* pos) {
     if (pos) std::memcpy(pos, host_u32_ + kRowsMax, n * 4);
 }
 
+// 64 rows of logits are 39 MB. Copied straight into pageable memory they took 4 ms, more than the step:
+// the runtime stages them through its own small buffer, with one thread that also takes the page faults
+// of a fresh destination. Here the transfers run through a ring of pinned slots and several threads
+// write each slot out while the next ones are in flight. Memory that is already pinned is copied to
+// directly, and so is less than a slot.
+void BatchDecoder::read_logits(int n, float* dst) {
+    const size_t bytes = (size_t)n * m_.cfg_.vocab * 4, slots = (bytes + kReadSlot - 1) / kReadSlot;
+    hipPointerAttribute_t at{};
+    const bool pinned = hipPointerGetAttributes(&at, dst) == hipSuccess && at.type == hipMemoryTypeHost;
+    (void)hipGetLastError();  // pageable memory may be reported as an error
+    if (pinned || slots < 2) {
+        QNE_HIP(hipMemcpyAsync(dst, logits_, bytes, hipMemcpyDeviceToHost, stream_));
+        sync();
+        return;
+    }
+    sync();  // the step, within its deadline; the transfers below are bounded
+    auto size = [&](size_t i) { return std::min(kReadSlot, bytes - i * kReadSlot); };
+    auto send = [&](size_t i) {
+        QNE_HIP(hipMemcpyAsync(host_read_ + (i % kReadSlots) * kReadSlot, (const uint8_t*)logits_ + i * kReadSlot, size(i),
+                               hipMemcpyDeviceToHost, stream_));
+        QNE_HIP(hipEventRecord(read_ev_[i % kReadSlots], stream_));
+    };
+    for (size_t i = 0; i < std::min<size_t>(kReadSlots, slots); i++) send(i);
+    const int threads = std::max(1, std::min(8, omp_get_max_threads()));
+    for (size_t i = 0; i < slots; i++) {
+        QNE_HIP(hipEventSynchronize(read_ev_[i % kReadSlots]));
+        const uint8_t* src = host_read_ + (i % kReadSlots) * kReadSlot;
+        uint8_t* out = (uint8_t*)dst + i * kReadSlot;
+        const size_t len = size(i), piece = (len / threads + 4095) / 4096 * 4096;
+#pragma omp parallel for num_threads(threads) schedule(static, 1)
+        for (int t = 0; t < threads; t++) {
+            const size_t a = std::min(len, t * piece), b = t + 1 == threads ? len : std::min(len, (t + 1) * piece);
+            std::memcpy(out + a, src + a, b - a);
+        }
+        if (i + kReadSlots < slots) send(i + kReadSlots);
+    }
+}
+
 void BatchDecoder::step(int n, const uint32_t* tokens, uint32_t* next, float* logits, size_t logits_cap) {
     if (n < 1 || n > max_rows_) throw Error(QNE_EINVAL, "rows must be 1..max_rows");
     const ModelConfig& c = m_.cfg_;
@@ -413,8 +461,8 @@ void BatchDecoder::step(int n, const uint32_t* tokens, uint32_t* next, float* lo
     }
     QNE_HIP(hipGraphLaunch(graph_for(n), stream_));
     QNE_HIP(hipMemcpyAsync(host_u32_, picks_, n * 4, hipMemcpyDeviceToHost, stream_));
-    if (logits) QNE_HIP(hipMemcpyAsync(logits, logits_, (size_t)n * c.vocab * 4, hipMemcpyDeviceToHost, stream_));
-    sync();
+    if (logits) read_logits(n, logits);
+    else sync();
     if (next) std::memcpy(next, host_u32_, n * 4);
 }
 

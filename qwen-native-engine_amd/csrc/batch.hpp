@@ -74,6 +74,7 @@ class BatchDecoder {
     void enqueue_step(int n);
     hipGraphExec_t graph_for(int n);
     void check_row(int row) const;
+    void read_logits(int n, float* dst);  // the first n rows into the caller's memory
     void sync(double steps = 1.0);  // waits with a deadline for `steps` batched steps
 
     Model& m_;
@@ -101,6 +102,10 @@ class BatchDecoder {
     int32_t* order_ = nullptr;  // the step's rows by decreasing position (attention partials' order)
     void* am_scratch_ = nullptr;  // per-row argmax partials
     uint32_t* host_u32_ = nullptr;  // pinned, 2 * 64 entries
+    static constexpr int kReadSlots = 4;
+    static constexpr size_t kReadSlot = 2u << 20;
+    uint8_t* host_read_ = nullptr;  // pinned, kReadSlots x kReadSlot bytes: logits on their way out
+    hipEvent_t read_ev_[kReadSlots] = {};
     double last_ms_ = 0.0;
     size_t last_steps_ = 0;
 };
