@@ -109,6 +109,9 @@ __global__ __launch_bounds__(256) void k_stage(const StageArgs a, int word_tiles
     else stage_columns(a, id % nx, id / nx);
 }
 
+// x alone (f16 weights have no words), few rows: no LDS, no divisions.
+__global__ __launch_bounds__(256) void k_stage_x(const StageArgs a) { stage_columns(a, blockIdx.x, blockIdx.y); }
+
 // Until at most n of the wave's vector-memory operations are outstanding (n wave-uniform; counts
 // past 31 wait for 31, which is only stricter).
 __device__ __forceinline__ void wait_vm_upto(int n) {
@@ -609,6 +612,7 @@ static void launch_stage(const GemmArgs& a, hipStream_t st) {
     }
     const int nx = (a.K + 255) / 256, wgs = nx * (a.mpad / 32);
     if (wgs >= 256) hipLaunchKernelGGL(k_stage<true>, dim3(tiles * pieces + wgs), dim3(256), 0, st, s, tiles, pieces);
+    else if (!tiles) hipLaunchKernelGGL(k_stage_x, dim3(nx, a.mpad), dim3(256), 0, st, s);
     else hipLaunchKernelGGL(k_stage<false>, dim3(tiles * pieces + nx * a.mpad), dim3(256), 0, st, s, tiles, pieces);
 }
 
