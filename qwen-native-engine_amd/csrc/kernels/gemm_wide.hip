@@ -17,10 +17,15 @@
 // the workgroups at the same LDS traffic per MFMA. Which form a column runs in depends on the matrix
 // and the caller's fixed row count, never on the rows of the call, so a row's sums are added in the
 // same order in every call.
-// Measured (2048 rows, K = 2048): N = 12288 with its epilogue 261 -> 203 us (206 GFLOP of MFMA, 1.0
-// PFLOP/s; a loop of these MFMAs alone on such data reaches 1.85), N = 8224 210 -> 157 us, N = 2048
-// 62 -> 43 us; K = 6144, N = 2048 136 -> 109 us. What is left: a workgroup's start and end are ~12 us
-// with its CU's matrix units idle, and a chunk (1.7 us) spends a third of its time around the barrier.
+// Measured (2048 rows, K = 2048; before: the 64-row form of batch.hip at two workgroups per CU): N =
+// 12288 with its epilogue 257 -> 203 us (206 GFLOP of MFMA, 1.0 PFLOP/s; a loop of these MFMAs alone, on
+// such data, reaches 1.85: the card's power limit), N = 8224 186 -> 160 us, N = 2048 60 -> 43 us, N = 2048
+// over the 2B model's K (2048, 4096, 6144) 105 -> 75 us. What is left: a workgroup's start and end are
+// ~10 us with its CU's matrix units idle, and a chunk takes 1.7 us for 1.1 of MFMA. Without the DMAs, the
+// LDS reads and the vector work together the loop is 11 % faster. Measured and not kept: two 4-wave
+// workgroups of 64 x 256 on a CU (N = 12288: 305 us), the halves of a workgroup one phase apart (+5 %),
+// raised wave priority around the MFMAs (+3 %), the DMAs early or late in a chunk (+1 %), no scheduling
+// fences, contiguous columns per XCD (no change).
 #include <algorithm>
 #include <type_traits>
 
@@ -217,7 +222,6 @@ __device__ __forceinline__ void wide_tile(const GemmArgs& a, WideLds<KG>& lds, c
     // one, and the DMAs of a later slot go out between the steps, so the matrix unit has work
     // throughout a phase. The empty asm statements pin each step's vector work to its step: left
     // alone, the compiler gathers it at the end of the chunk and copies grp to keep it alive.
-    // Measured and not kept: the workgroup's second half one phase behind the first (5 % slower).
     int slot = 0, next_slot = kWideRing - 1;
     float16_t grp[2][2] = {};       // [column tile][row tile]
     float sc[2] = {};

@@ -1,5 +1,5 @@
 // Chunked prefill on the batched GEMM: Model::prefill_chunk (kernels/src/model.rs:349-372) runs
-// the prompt up to 512 tokens per pass, as the reference's prefill_batched runs 16
+// the prompt up to 2048 tokens per pass, as the reference's prefill_batched runs 16
 // (kernels/src/batch.rs). A pass's tokens are the rows of one pass through the layers: every
 // projection is one MFMA GEMM over the pass (in tiles of 64 rows, so the weights stream once per
 // pass), attention appends the pass's K/V and each token attends positions up to its own (causal by
