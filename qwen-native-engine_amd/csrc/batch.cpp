@@ -410,14 +410,14 @@ void BatchDecoder::row_state(int n, uint32_t* tokens, uint32_t* pos) {
 // 64 rows of logits are 39 MB. Copied straight into pageable memory they took 4 ms, more than the step:
 // the runtime stages them through its own small buffer, with one thread that also takes the page faults
 // of a fresh destination. Here the transfers run through a ring of pinned slots and several threads
-// write each slot out while the next ones are in flight. Memory that is already pinned is copied to
-// directly, and so is less than a slot.
+// write each slot out while the next ones are in flight. Memory that the runtime knows (pinned, managed)
+// is copied to directly, and so is less than a slot.
 void BatchDecoder::read_logits(int n, float* dst) {
     const size_t bytes = (size_t)n * m_.cfg_.vocab * 4, slots = (bytes + kReadSlot - 1) / kReadSlot;
     hipPointerAttribute_t at{};
-    const bool pinned = hipPointerGetAttributes(&at, dst) == hipSuccess && at.type == hipMemoryTypeHost;
+    const bool pageable = hipPointerGetAttributes(&at, dst) != hipSuccess || at.type == hipMemoryTypeUnregistered;
     (void)hipGetLastError();  // pageable memory may be reported as an error
-    if (pinned || slots < 2) {
+    if (!pageable || slots < 2) {
         QNE_HIP(hipMemcpyAsync(dst, logits_, bytes, hipMemcpyDeviceToHost, stream_));
         sync();
         return;

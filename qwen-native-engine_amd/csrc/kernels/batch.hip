@@ -140,8 +140,8 @@ __device__ __forceinline__ void wait_vm_upto(int n) {
 // of one W tile read the same W chunks, which the MALL serves after the first.
 // Epilogues: partials (split-K, or an epilogue the GEMM does not apply); `direct` (one split: store
 // or residual add); `fuse` 1 (one split, SwiGLU): tiles [0, TW / 2) are gate rows and [TW / 2, TW)
-// the matching up rows (n_out further), and the workgroup writes silu(gate) * up and stages it as
-// the next GEMM's operand, exactly as k_gemm_reduce does with one split.
+// the matching up rows (n_out further), and the workgroup writes silu(gate) * up, exactly as
+// k_gemm_reduce does with one split.
 template <int KIND, int WAVES, int D, int DW, int CF>
 __global__ __launch_bounds__(64 * (WAVES + DW)) void k_gemm(const GemmArgs a) {
     constexpr int TW = WAVES * CF;                                  // 32-row W tiles per workgroup
@@ -363,8 +363,8 @@ __global__ __launch_bounds__(64 * (WAVES + DW)) void k_gemm(const GemmArgs a) {
         return;
     }
     // fused SwiGLU: the up tiles go through LDS ([row][column of the workgroup's gate columns]),
-    // the gate tiles' lanes form silu(g / rms) * (u / rms) in place, then every wave stages whole
-    // 64-column chunks of rows (lanes = columns), as the reduce does
+    // the gate tiles' lanes form silu(g / rms) * (u / rms) in place, then every wave stores whole
+    // 64-column chunks of rows (lanes = columns)
     constexpr int kCols = TW / 2 * 32;  // output columns of the workgroup
     static_assert(kCols % kChunk == 0 && (kBM * kCols + kBM) * 4 <= D * kSlot, "fused SwiGLU tile");
     float* sv = sinv + kBM;  // [kBM][kCols]
@@ -400,13 +400,11 @@ __global__ __launch_bounds__(64 * (WAVES + DW)) void k_gemm(const GemmArgs a) {
     __syncthreads();
     if (!computes) return;
     constexpr int nck = kCols / kChunk;
-    const size_t tile_bytes = (size_t)(a.n_out / kChunk) * kChunkBytes;
     for (int it = w; it < min(rows, kBM) * nck; it += WAVES) {  // wave-uniform
         const int r = it / nck, ch = it % nck;
         const int c = blockIdx.x * kCols + ch * kChunk + lane;
         const float v = sv[r * kCols + ch * kChunk + lane];
-        if (a.y) store_through(a.y + (size_t)(kBM * mt + r) * a.y_stride + c, v);
-        if (a.frag_out) emit_x(a.frag_out, tile_bytes, kBM * mt + r, c, v, a.gain_out ? a.gain_out[c] : 1.0f, a.order_out, lane);
+        store_through(a.y + (size_t)(kBM * mt + r) * a.y_stride + c, v);
     }
 }
 
@@ -640,7 +638,7 @@ void launch_gemm(GemmArgs a, hipStream_t st) {
     const bool one = a.fuse == 0 && a.kind == KIND_Q4 && !dma_waves && a.splits == 1 && !a.partials_only && !few;
     a.fuse = 0;
     if (one && a.epi == EPI_SWIGLU && a.N == 2 * a.n_out && a.n_out % (32 * waves / 2) == 0 && a.K <= 64 * kChunk &&
-        (a.y || a.frag_out))
+        (wide ? a.y || a.frag_out : a.y && !a.frag_out))  // only the wide form stages a SwiGLU
         a.fuse = 1;
     // store or residual add staged as the next operand (with a normed input its 1 / rms needs K <= 4096)
     else if (one && wide && a.epi != EPI_SWIGLU && a.frag_out && a.n_out == a.N && a.N % kChunk == 0 &&
