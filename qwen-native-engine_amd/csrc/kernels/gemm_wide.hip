@@ -5,11 +5,15 @@
 // per chunk, and left the matrix units idle for 70 % of the time. Here:
 //  - a wave computes 64 rows x 64 columns, so 18 KiB of LDS reads feed 32 MFMAs (17 KiB fed 16), and
 //    a weight is dequantised once per 64 rows;
-//  - the weights enter the matrix units as q - 8 and the zero points' share, sum over the chunks of
-//    s (8 - z) sum x, is the accumulators' first value: one small product on the bf16 matrix units
-//    (f32 operands as three bf16 terms, six products, to 2^-24), before the first chunk. A chunk then
-//    costs one fma per output value instead of two, and no row sums from LDS; the error against 64
-//    bits is 0.6 of what it was (the products no longer carry the zero points);
+//  - the weights enter the matrix units as q - r, r the integer in 0..15 nearest the group's zero point z,
+//    and what is left of the zero points, sum over the chunks of s (r - z) sum x, is the accumulators'
+//    first value: one small product on the bf16 matrix units (f32 operands as three bf16 terms, six
+//    products, to 2^-24), before the first chunk. A chunk then costs one fma per output value instead of
+//    two, and no row sums from LDS. With r the products and the first value have the size of the sums
+//    themselves, wherever the zero points lie. Error against 64 bits (2-norm, 1024 x 2048 x 1024, the
+//    64-row form / this one): zeros 7.5, codes 0..15 2.0e-7 / 1.0e-7, zeros 0, codes 0..1 1.2e-7 / 1.0e-7,
+//    zeros 15, codes 14..15 2.1e-6 / 1.0e-7 (r = 8 for every group: 1.0e-7, 1.2e-6, 1.1e-6). A chain of 32
+//    chunks (K = 2048 in one split) adds a little: 1.3e-7, and 1.8e-7 for zeros far outside 0..15;
 //  - the epilogue stages the next GEMM's operand 16 bytes a lane.
 // A workgroup is 8 waves over 256 columns. 128 rows (KG = 1): 2 x 4 waves, every wave takes every
 // chunk. 64 rows (KG = 2): 4 waves across, and the two halves of the workgroup take the even and the
@@ -56,6 +60,9 @@ struct Bf3 {
         t[2][i] = (__bf16)(r - (float)b);
     }
 };
+
+// s (r - z): what the products of q - r leave of a group's zero point.
+__device__ __forceinline__ float zero_rest(uint32_t szw) { return lo_h(szw) * (zero_int(szw).value() - hi_h(szw)); }
 
 constexpr int kWideCols = 256;  // W rows (output columns) of a workgroup
 constexpr int kWideWaves = 8;
@@ -123,23 +130,25 @@ __device__ __forceinline__ void wide_tile(const GemmArgs& a, WideLds<KG>& lds, c
         woff[u] = (uint32_t)(min(wrow0(w) + row, a.N - 1) - tile0) * (a.K / 2) + 16 * (piece & 1);
     }
     auto group = [&](int c) -> int { return cpg == 1 ? c : (int)((unsigned)c / (unsigned)cpg); };
-    // DMA u (of kPer) of slot j
+    // DMA u (of kPer) of slot j: the words, x, W
     const uint32_t ring_lds = lds_address(ring);
     auto issue = [&](int j, int slot, int u) {
         const uint32_t base = ring_lds + slot * kSlot;
         const int c = c0 + KG * j;
-        if (u < 4) {
-            dma16_at(xtile + (size_t)min(c + (KG == 2 ? half : 0), c1 - 1) * kChunkBytes + 4096 * nw + 1024 * u, 16 * lane,
-                     base + 2 * kFragBytes * half + 4096 * nw + 1024 * u);
-        } else if (u < 4 + KG) {
+        if (u == 0) {
+            if (lane < 8 * KG) {
+                if (KG == 1) dma16_at(szbase + (size_t)group(c) * 128, 16 * lane, base + kX + kW + 128 * w);
+                else dma16_at(szbase, (uint32_t)group(min(c + (lane >> 3), c1 - 1)) * 128 + 16 * (lane & 7), base + kX + kW + KG * 128 * w);
+            }
+        } else if (u < 5) {
+            const int o = 4096 * nw + 1024 * (u - 1);
+            dma16_at(xtile + (size_t)min(c + (KG == 2 ? half : 0), c1 - 1) * kChunkBytes + o, 16 * lane, base + 2 * kFragBytes * half + o);
+        } else {
             if (KG == 1) dma16_at(wbase + (size_t)c * 32, woff[0], base + kX + 1024 * w);
-            else dma16_at(wbase, woff[u - 4] + min(c + wchunk[u - 4], c1 - 1) * 32, base + kX + KG * 1024 * w + 1024 * (u - 4));
-        } else if (lane < 8 * KG) {
-            if (KG == 1) dma16_at(szbase + (size_t)group(c) * 128, 16 * lane, base + kX + kW + 128 * w);
-            else dma16_at(szbase, (uint32_t)group(min(c + (lane >> 3), c1 - 1)) * 128 + 16 * (lane & 7), base + kX + kW + KG * 128 * w);
+            else dma16_at(wbase, woff[u - 5] + min(c + wchunk[u - 5], c1 - 1) * 32, base + kX + KG * 1024 * w + 1024 * (u - 5));
         }
     };
-    // acc's first value: sum over this wave's chunks of s (8 - z) sum x. The chunks are the contraction,
+    // acc's first value: sum over this wave's chunks of s (r - z) sum x. The chunks are the contraction,
     // 16 at a time; a batch's loads are in flight together, the first batch's (and the first sums of
     // x^2) ahead of the first chunks' DMAs.
     const int nmine = (c1 - cfirst + KG - 1) / KG;
@@ -202,7 +211,7 @@ __device__ __forceinline__ void wide_tile(const GemmArgs& a, WideLds<KG>& lds, c
 #pragma unroll
             for (int t = 0; t < 2; t++) {
                 xa[t].set(i, live ? xv[t][i] : 0.0f);
-                wb[t].set(i, live ? lo_h(sz[t][i]) * (8.0f - hi_h(sz[t][i])) : 0.0f);
+                wb[t].set(i, live ? zero_rest(sz[t][i]) : 0.0f);
             }
         }
         if (b + 16 < nmine) load_sums(b + 16);
@@ -218,26 +227,30 @@ __device__ __forceinline__ void wide_tile(const GemmArgs& a, WideLds<KG>& lds, c
     }
 
     // A chunk runs as two phases, one per 32-row tile, of four k-steps: the first dequantises the
-    // weights and keeps them for the second. The scaled sums of a phase are added during the next
+    // weights and keeps them for the second, which reads the next chunk's words and rounds its zero
+    // points (at the start of their own chunk they delay its first product: N = 12288 201 -> 205 us). The scaled sums of a phase are added during the next
     // one, and the DMAs of a later slot go out between the steps, so the matrix unit has work
     // throughout a phase. The empty asm statements pin each step's vector work to its step: left
     // alone, the compiler gathers it at the end of the chunk and copies grp to keep it alive.
     int slot = 0, next_slot = kWideRing - 1;
     float16_t grp[2][2] = {};       // [column tile][row tile]
     float sc[2] = {};
+    uint32_t szw[2];                // this wave's words of the chunk that comes next
+    ZeroInt zi[2];
+    auto read_words = [&](int at) {
+        const uint8_t* wsz = ring + at * kSlot + kX + kW + 2 * nw * KG * 128 + (KG == 2 ? 128 * half : 0) + 4 * l32;
+#pragma unroll
+        for (int cf = 0; cf < 2; cf++) szw[cf] = *(const uint32_t*)(wsz + cf * KG * 128);
+    };
     const int piece = KG == 1 ? hf : (2 * half + hf) ^ ((l32 >> 2) & 3);
     auto chunk = [&](int j, auto sends) {
         const uint8_t* xs = ring + slot * kSlot + 2 * kFragBytes * half;
         const uint8_t* ws = ring + slot * kSlot + kX + 2 * nw * KG * 1024;
-        const uint8_t* wsz = ring + slot * kSlot + kX + kW + 2 * nw * KG * 128 + (KG == 2 ? 128 * half : 0) + 4 * l32;
         uint4 wq[2];
-        uint32_t szw[2];
         half8_t b[2][4];
 #pragma unroll
         for (int cf = 0; cf < 2; cf++) wq[cf] = *(const uint4*)(ws + cf * KG * 1024 + (l32 * kPieces + piece) * 16);
         half8_t ah = *(const half8_t*)(xs + frag_offset(0, 0, lane)), al = *(const half8_t*)(xs + kFragBytes + frag_offset(0, 0, lane));
-#pragma unroll
-        for (int cf = 0; cf < 2; cf++) szw[cf] = *(const uint32_t*)(wsz + cf * KG * 128);
 #pragma unroll
         for (int p = 0; p < 8; p++) {
             const int rt = p >> 2, s = p & 3, np = p + 1;
@@ -248,7 +261,7 @@ __device__ __forceinline__ void wide_tile(const GemmArgs& a, WideLds<KG>& lds, c
             }
             if (rt == 0) {
 #pragma unroll
-                for (int cf = 0; cf < 2; cf++) b[cf][s] = nibbles8_signed(s == 0 ? wq[cf].x : s == 1 ? wq[cf].y : s == 2 ? wq[cf].z : wq[cf].w);
+                for (int cf = 0; cf < 2; cf++) b[cf][s] = nibbles8(s == 0 ? wq[cf].x : s == 1 ? wq[cf].y : s == 2 ? wq[cf].z : wq[cf].w, zi[cf]);
             }
             const float16_t zero = {};
 #pragma unroll
@@ -258,6 +271,11 @@ __device__ __forceinline__ void wide_tile(const GemmArgs& a, WideLds<KG>& lds, c
             if (p == 4) {
 #pragma unroll
                 for (int cf = 0; cf < 2; cf++) sc[cf] = lo_h(szw[cf]);
+                read_words(slot + 1 == kWideRing ? 0 : slot + 1);
+            }
+            if (p == 7) {
+#pragma unroll
+                for (int cf = 0; cf < 2; cf++) zi[cf] = zero_int(szw[cf]);
             }
 #pragma unroll
             for (int cf = 0; cf < 2; cf++)
@@ -275,11 +293,16 @@ __device__ __forceinline__ void wide_tile(const GemmArgs& a, WideLds<KG>& lds, c
         slot = slot + 1 == kWideRing ? 0 : slot + 1;
         next_slot = next_slot + 1 == kWideRing ? 0 : next_slot + 1;
     };
-    // A wave whose columns all lie past N only sends. At the barrier every part of slot j has landed,
-    // and every wave is done with slot j - 1.
+    // A wave whose columns all lie past N only sends. At the barrier every part of slot j and the words
+    // of slot j + 1 (its first DMA) have landed, and every wave is done with slot j - 1.
     const bool dead = wrow0(2 * nw) >= a.N;
+    wait_vm<kPer - 1>();
+    __syncthreads();
+    read_words(0);
+#pragma unroll
+    for (int cf = 0; cf < 2; cf++) zi[cf] = zero_int(szw[cf]);
     for (int j = 0; j < iters - (kWideRing - 1); j++) {
-        wait_vm<kPer>();
+        wait_vm<kPer - 1>();
         __syncthreads();
         if (dead) {
 #pragma unroll
@@ -290,7 +313,7 @@ __device__ __forceinline__ void wide_tile(const GemmArgs& a, WideLds<KG>& lds, c
         }
     }
     if (iters > 1) {
-        wait_vm<kPer>();
+        wait_vm<kPer - 1>();
         __syncthreads();
         if (!dead) chunk(iters - 2, std::false_type());
     }
@@ -462,9 +485,9 @@ __global__ __launch_bounds__(64 * kWideWaves) void k_gemm_short(const GemmArgs a
     struct Operands {
         half8_t h[4], l[4];
         uint4 w[CT];
-        uint32_t sz[kWideWaves];
+        uint32_t wz[CT], sz[kWideWaves];
     } ops[2];  // of two rounds: one computed, the next one's loads in flight
-    auto load = [&](Operands& o, int r) {  // round r: this wave's chunk, and the scales of all of them
+    auto load = [&](Operands& o, int r) {  // round r: this wave's chunk, and the scales of its registers in all of them
         const int c = c0 + min(8 * r + w, nch - 1);
         const uint8_t* xs = xtile + (size_t)c * kChunkBytes;
 #pragma unroll
@@ -473,7 +496,10 @@ __global__ __launch_bounds__(64 * kWideWaves) void k_gemm_short(const GemmArgs a
             o.l[s] = *(const half8_t*)(xs + kFragBytes + frag_offset(s, rt, lane));
         }
 #pragma unroll
-        for (int t = 0; t < CT; t++) o.w[t] = *(const uint4*)(wrow[t] + (size_t)c * 32);
+        for (int t = 0; t < CT; t++) {
+            o.w[t] = *(const uint4*)(wrow[t] + (size_t)c * 32);
+            o.wz[t] = szt[t][(size_t)group(c) * 32];
+        }
         const uint32_t* sp = CT == 1 || own_t == 0 ? szt[0] : szt[CT - 1];
 #pragma unroll
         for (int k = 0; k < kWideWaves; k++) o.sz[k] = sp[(size_t)group(c0 + min(8 * r + k, nch - 1)) * 32];
@@ -501,7 +527,7 @@ __global__ __launch_bounds__(64 * kWideWaves) void k_gemm_short(const GemmArgs a
             for (int i = 0; i < 8; i++) {
                 const bool live = b + 8 * hf + i < nmine;
                 xa.set(i, live ? xv[i] : 0.0f);
-                wb.set(i, live ? lo_h(sv[i]) * (8.0f - hi_h(sv[i])) : 0.0f);
+                wb.set(i, live ? zero_rest(sv[i]) : 0.0f);
             }
 #pragma unroll
             for (int p = 2; p >= 0; p--)
@@ -521,11 +547,14 @@ __global__ __launch_bounds__(64 * kWideWaves) void k_gemm_short(const GemmArgs a
     const int rounds = (nch + kWideWaves - 1) / kWideWaves;
     auto round = [&](const Operands& cur, int r) {
         float16_t grp[CT] = {};
+        ZeroInt zi[CT];
+#pragma unroll
+        for (int t = 0; t < CT; t++) zi[t] = zero_int(cur.wz[t]);
 #pragma unroll
         for (int s = 0; s < 4; s++) {
             half8_t b[CT];
 #pragma unroll
-            for (int t = 0; t < CT; t++) b[t] = nibbles8_signed(s == 0 ? cur.w[t].x : s == 1 ? cur.w[t].y : s == 2 ? cur.w[t].z : cur.w[t].w);
+            for (int t = 0; t < CT; t++) b[t] = nibbles8(s == 0 ? cur.w[t].x : s == 1 ? cur.w[t].y : s == 2 ? cur.w[t].z : cur.w[t].w, zi[t]);
 #pragma unroll
             for (int t = 0; t < CT; t++) grp[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(cur.h[s], b[t], grp[t], 0, 0, 0);
 #pragma unroll

@@ -101,6 +101,30 @@ def test_gemm_wide_forms(rows, k, group, M, epi):
     assert rel_err(got, want) < 2e-5
 
 
+@pytest.mark.parametrize("zero,codes", [(7.5, (0, 15)), (0.0, (0, 1)), (0.0, (0, 3)), (15.0, (14, 15)), (3.49, (0, 7)),
+                                        (-20.0, (0, 15)), (40.0, (0, 15))])
+@pytest.mark.parametrize("rows,M", [(1024, 1024), (12288, 300)])  # four splits of 8 chunks; one of 32
+def test_gemm_wide_zero_points(zero, codes, rows, M):
+    """A pass's GEMM over weights that are centred on zero, one-sided, or shifted: the precision does not
+    depend on where the zero points lie. Bar: x as two f16 halves keeps 22 bits (2^-23 = 1.2e-7 of a
+    product at most), the f32 sums over 64 columns and up to 32 chunks each round to 2^-24 of a partial
+    sum, about 1e-7 over a chain; 2.5e-7 in the 2-norm (measured 1.0e-7 to 1.6e-7)."""
+    k, group = 2048, 64
+    rng = np.random.default_rng(rows + M)
+    q = rng.integers(codes[0], codes[1] + 1, size=(rows, k), dtype=np.uint8)
+    s = rng.uniform(0.002, 0.03, size=(rows, k // group)).astype(np.float16)
+    z = np.full((rows, k // group), zero, np.float16)
+    X = rng.normal(size=(M, k)).astype(np.float32)
+    W = ((q.reshape(rows, -1, group) - z[..., None].astype(np.float64)) * s[..., None].astype(np.float64)).reshape(rows, k)
+    want = X.astype(np.float64) @ W.T
+    dw, dsz, dx = to_dev(q[:, 0::2] | (q[:, 1::2] << 4)), to_dev(np.stack([s, z], -1).view(np.uint16)), to_dev(X)
+    got = D.zeros((M, rows), np.float32)
+    Q.gemm(Q.MAT_Q4, dw.data_ptr(), dsz.data_ptr(), rows, k, group, dx.data_ptr(), k, M, got.data_ptr(), rows)
+    D.sync()
+    err = np.linalg.norm(got.numpy() - want) / np.linalg.norm(want)
+    assert err < 2.5e-7, err
+
+
 @pytest.mark.parametrize("kind,group", [(Q.MAT_Q4, 64), (Q.MAT_F16, 0)])
 def test_gemm_one_split_direct_epilogue(kind, group):
     """More than 512 tiles of 128 rows: one split, the GEMM applies 1 / rms and the epilogue itself
