@@ -30,7 +30,8 @@ __device__ __forceinline__ int frag_offset(int s, int mt, int lane) { return ((s
 
 // Writes one value of the x operand of a GEMM: row r, column c, value v (times gain g). The 64
 // lanes of the calling wave hold the 64 columns of one chunk of row r (all lanes call it), so the
-// chunk's sums of hi + lo and of v^2 are wave sums. q4order: the column order of the q4 GEMM's B
+// chunk's sums of hi + lo and of v^2 are wave sums. lo is what hi leaves of the unrounded product
+// v g (one fma). q4order: the column order of the q4 GEMM's B
 // operand within each 8 columns, [0, 4, 1, 5, 2, 6, 3, 7] (nibbles8); else natural. Rows come in
 // tiles of 64: tile r / 64 of the operand starts tile_bytes (the K / 64 chunks of one tile) after
 // the previous one.
@@ -39,7 +40,7 @@ __device__ __forceinline__ void emit_x(uint8_t* __restrict__ frag, size_t tile_b
 #pragma clang fp contract(off)  // the sums' rounding is the same wherever an operand is staged
     const float xg = v * g;
     const float hi = (float)(_Float16)xg;
-    const float lo = (float)(_Float16)(xg - hi);
+    const float lo = (float)(_Float16)fmaf(v, g, -hi);
     const int chunk = c / kChunk, kk = c % kChunk, hf = kk / 32, st = (kk % 32) / 8, i = kk % 8;
     const int slot = q4order ? 2 * (i % 4) + i / 4 : i;
     const int rr = r & (kBM - 1);
@@ -72,7 +73,7 @@ __device__ __forceinline__ void emit_x_rows(uint8_t* __restrict__ frag, size_t t
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             const float xg = v[8 * s + i] * g[8 * s + i];
-            const _Float16 h = (_Float16)xg, l = (_Float16)(xg - (float)h);
+            const _Float16 h = (_Float16)xg, l = (_Float16)fmaf(v[8 * s + i], g[8 * s + i], -(float)h);
             hi[i] = __builtin_bit_cast(uint16_t, h);
             lo[i] = __builtin_bit_cast(uint16_t, l);
             xt[i] = (float)h + (float)l;

@@ -101,6 +101,45 @@ def test_gemm_wide_forms(rows, k, group, M, epi):
     assert rel_err(got, want) < 2e-5
 
 
+def fused_split(v, g):
+    """hi + lo of v g as the operand holds it, lo from the unrounded product, and from the rounded one."""
+    exact = v.astype(np.float64) * g.astype(np.float64)
+    rounded = exact.astype(np.float32)
+    hi = rounded.astype(np.float16).astype(np.float64)
+    return [hi + (p - hi).astype(np.float32).astype(np.float16).astype(np.float64) for p in (exact, rounded)]
+
+
+@pytest.mark.parametrize("kind", [Q.MAT_Q4, Q.MAT_F16])
+@pytest.mark.parametrize("k,M", [(64, 3), (2048, 1024)])  # staged a value a lane, and 32 rows of a chunk a wave
+def test_gemm_operand_keeps_the_unrounded_product(kind, k, M):
+    """x times the norm's gain is split into f16 halves from its unrounded product. x is 1.5 in 3 of 8
+    columns and 0.5 in the others (its mean square is 1, so with eps 0 the factor 1 / rms is exactly 1), the
+    gains are ones where the two roundings differ, and the matrix picks columns: results are exact."""
+    rng = np.random.default_rng(k)
+    g = (1 + rng.integers(0, 1 << 23, size=1 << 16) / (1 << 23)).astype(np.float32)
+    fused, split = fused_split(np.full(g.size, 1.5, np.float32), g)
+    g = g[(fused != split) & (fused.astype(np.float32) == fused)]
+    big = np.arange(k) % 8 < 3
+    assert g.size >= 64
+    G = np.ones(k, np.float32)
+    G[big] = g[np.arange(big.sum()) % g.size]
+    cols = np.flatnonzero(big)[np.linspace(0, big.sum() - 1, 24).astype(int)]
+    X = np.where(big, 1.5, 0.5).astype(np.float32) * np.where(np.arange(M) % 2, -1, 1).astype(np.float32)[:, None]
+    want = fused_split(X[:, cols], np.broadcast_to(G[cols], (M, 24)))[0].astype(np.float32)
+    one = np.zeros((24, k), np.uint8)
+    one[np.arange(24), cols] = 1
+    if kind == Q.MAT_Q4:
+        w = one[:, 0::2] | (one[:, 1::2] << 4)
+        dsz = to_dev(np.tile(np.array([1, 0], np.float16).view(np.uint16), (24, k // 64)))  # scale 1, zero 0
+    else:
+        w, dsz = one.astype(np.float16).view(np.uint16), None
+    dw, dx, dg, dy = to_dev(w), to_dev(X), to_dev(G), D.zeros((M, 24), np.float32)
+    Q.gemm(kind, dw.data_ptr(), dsz.data_ptr() if dsz else 0, 24, k, 64, dx.data_ptr(), k, M, dy.data_ptr(), 24,
+           norm=dg.data_ptr(), eps=0.0)
+    D.sync()
+    assert np.array_equal(dy.numpy(), want)
+
+
 @pytest.mark.parametrize("zero,codes", [(7.5, (0, 15)), (0.0, (0, 1)), (0.0, (0, 3)), (15.0, (14, 15)), (3.49, (0, 7)),
                                         (-20.0, (0, 15)), (40.0, (0, 15))])
 @pytest.mark.parametrize("rows,M", [(1024, 1024), (12288, 300)])  # four splits of 8 chunks; one of 32
