@@ -45,9 +45,8 @@ __device__ __forceinline__ float lane_xor16(float v, int lane) {
     return __uint_as_float((lane & 16) ? p[0] : p[1]);
 }
 // Sum over the 64 lanes of a wave with DPP and permlane swaps; every lane receives the total.
-__device__ __forceinline__ float wave_sum_dpp(float v) {
+__device__ __forceinline__ float wave_sum_dpp_pairs(float v) {  // v: the sum of the lane's pair
     const int lane = (int)__lane_id();
-    v += QNE_DPP(v, kDppXor1);
     v += QNE_DPP(v, kDppXor2);
     v += QNE_DPP(v, kDppHalfMirror);
     v += QNE_DPP(v, kDppMirror);
@@ -55,6 +54,7 @@ __device__ __forceinline__ float wave_sum_dpp(float v) {
     v += lane_xor32(v, lane);
     return v;
 }
+__device__ __forceinline__ float wave_sum_dpp(float v) { return wave_sum_dpp_pairs(v + QNE_DPP(v, kDppXor1)); }
 
 // Sum over each half (32 lanes) of a wave; every lane receives its half's total.
 __device__ __forceinline__ float half_sum_dpp(float v, int lane) {

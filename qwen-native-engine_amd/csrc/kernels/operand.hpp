@@ -31,7 +31,7 @@ __device__ __forceinline__ int frag_offset(int s, int mt, int lane) { return ((s
 // Writes one value of the x operand of a GEMM: row r, column c, value v (times gain g). The 64
 // lanes of the calling wave hold the 64 columns of one chunk of row r (all lanes call it), so the
 // chunk's sums of hi + lo and of v^2 are wave sums. lo is what hi leaves of the unrounded product
-// v g (one fma). q4order: the column order of the q4 GEMM's B
+// v g (one fma), and a pair's squares are added with one rounding. q4order: the column order of the q4 GEMM's B
 // operand within each 8 columns, [0, 4, 1, 5, 2, 6, 3, 7] (nibbles8); else natural. Rows come in
 // tiles of 64: tile r / 64 of the operand starts tile_bytes (the K / 64 chunks of one tile) after
 // the previous one.
@@ -48,7 +48,8 @@ __device__ __forceinline__ void emit_x(uint8_t* __restrict__ frag, size_t tile_b
     uint8_t* dst = tile + frag_offset(st, rr >> 5, 32 * hf + (rr & 31)) + 2 * slot;
     *(uint16_t*)dst = __builtin_bit_cast(uint16_t, (_Float16)hi);
     *(uint16_t*)(dst + kFragBytes) = __builtin_bit_cast(uint16_t, (_Float16)lo);
-    const float xs = wave_sum_dpp(hi + lo), ss = wave_sum_dpp(v * v);
+    const float sq = v * v;
+    const float xs = wave_sum_dpp(hi + lo), ss = wave_sum_dpp_pairs(fmaf(v, v, QNE_DPP(sq, kDppXor1)));
     if (lane == 0) {
         float* sums = (float*)tile;
         sums[kXsumOff / 4 + rr] = xs;
@@ -69,7 +70,7 @@ __device__ __forceinline__ void emit_x_rows(uint8_t* __restrict__ frag, size_t t
 #pragma unroll
     for (int s = 0; s < 4; s++) {
         uint16_t hi[8], lo[8];
-        float xt[8], st[8];
+        float xt[8], st[4];
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             const float xg = v[8 * s + i] * g[8 * s + i];
@@ -77,10 +78,16 @@ __device__ __forceinline__ void emit_x_rows(uint8_t* __restrict__ frag, size_t t
             hi[i] = __builtin_bit_cast(uint16_t, h);
             lo[i] = __builtin_bit_cast(uint16_t, l);
             xt[i] = (float)h + (float)l;
-            st[i] = v[8 * s + i] * v[8 * s + i];
+        }
+        // emit_x's lane 0 sees the first four columns from their even lanes and the next four, mirrored, from
+        // their odd ones: that lane's square is the unrounded one
+#pragma unroll
+        for (int p = 0; p < 4; p++) {
+            const int own = 2 * p + p / 2, other = own ^ 1;
+            st[p] = fmaf(v[8 * s + own], v[8 * s + own], v[8 * s + other] * v[8 * s + other]);
         }
         xs[s] = ((xt[0] + xt[1]) + (xt[2] + xt[3])) + ((xt[4] + xt[5]) + (xt[6] + xt[7]));
-        ss[s] = ((st[0] + st[1]) + (st[2] + st[3])) + ((st[4] + st[5]) + (st[6] + st[7]));
+        ss[s] = (st[0] + st[1]) + (st[2] + st[3]);
         uint32_t hw[4], lw[4];
 #pragma unroll
         for (int p = 0; p < 4; p++) {  // word p: slots 2 p, 2 p + 1 (q4 order: columns p, p + 4)

@@ -140,6 +140,28 @@ def test_gemm_operand_keeps_the_unrounded_product(kind, k, M):
     assert np.array_equal(dy.numpy(), want)
 
 
+@pytest.mark.parametrize("k,M", [(64, 3), (2048, 1024)])
+def test_gemm_operand_adds_a_pairs_squares_with_one_rounding(k, M):
+    """The norm's sum of x^2 takes a pair of columns as fma(a, a, b^2), in both staging forms. Rows hold one
+    pair and a one; the matrix picks the one, so the result is 1 / rms, and the pairs are ones for which the
+    sum's rounding shows in it."""
+    f = np.float32
+    rng = np.random.default_rng(k)
+    a, b = rng.uniform(64, 128, size=(2, 1 << 16)).astype(f)
+    low = b * b
+    fused, split = ((s + f(1)) / f(k) for s in ((a.astype(np.float64) ** 2 + low).astype(f), a * a + low))
+    keep = np.flatnonzero(f(1) / np.sqrt(fused) != f(1) / np.sqrt(split))[:M]
+    keep = np.resize(keep, M)
+    X = np.zeros((M, k), f)
+    X[:, 0], X[:, 1], X[:, 8] = a[keep], b[keep], 1
+    w = np.zeros((1, k), np.float16)
+    w[0, 8] = 1
+    dw, dx, dg, dy = to_dev(w.view(np.uint16)), to_dev(X), to_dev(np.ones(k, f)), D.zeros((M, 1), f)
+    Q.gemm(Q.MAT_F16, dw.data_ptr(), 0, 1, k, 0, dx.data_ptr(), k, M, dy.data_ptr(), 1, norm=dg.data_ptr(), eps=0.0)
+    D.sync()
+    assert np.array_equal(dy.numpy()[:, 0], f(1) / np.sqrt(fused[keep]))
+
+
 @pytest.mark.parametrize("zero,codes", [(7.5, (0, 15)), (0.0, (0, 1)), (0.0, (0, 3)), (15.0, (14, 15)), (3.49, (0, 7)),
                                         (-20.0, (0, 15)), (40.0, (0, 15))])
 @pytest.mark.parametrize("rows,M", [(1024, 1024), (12288, 300)])  # four splits of 8 chunks; one of 32
