@@ -75,6 +75,7 @@ constexpr int kWideRing = 3;    // slots: one computed, two in flight
 template <int KG>
 struct WideLds {
     static constexpr int kRows = 128 / KG;
+    static constexpr int kSquares = 4;                // classes of 64 chunks
     static constexpr int kX = 2 * 2 * kFragBytes;
     static constexpr int kW = KG * 8 * 1024;
     static constexpr int kSz = KG * 8 * 128;
@@ -83,7 +84,7 @@ struct WideLds {
     static constexpr int kRing = kWideRing * kSlot > kRows * kOutStride * 4 ? kWideRing * kSlot : kRows * kOutStride * 4;
     __attribute__((aligned(16))) uint8_t ring[kRing];
     float sinv[kRows];
-    float parts[512];                                 // partial sums of the rows' x^2
+    float parts[kSquares][512];                       // partial sums of the rows' x^2
 };
 
 // Column tile bx, row tile bz (of 128 / KG rows), split by: chunks [by cps, (by + 1) cps).
@@ -170,37 +171,43 @@ __device__ __forceinline__ void wide_tile(const GemmArgs& a, WideLds<KG>& lds, c
         }
     };
     load_sums(0);
-    // A row's sum of x^2: thread t of the row's 4 KG takes the chunks t + 4 KG k (a batch of 64), and
-    // the tree below adds them in the order of row_inv_rms (a butterfly over 64 lanes, lane = chunk).
+    // A row's sum of x^2 in the order of row_inv_rms, whose thread c of 256 takes chunks c, c + 256, .. and
+    // whose four waves of 64 threads are a butterfly each: here class q of 64 threads is thread t of the
+    // row's 4 KG with the chunks 64 q + t + 4 KG k, and the trees below are the butterfly.
     const bool norm = a.norm && (a.direct || a.fuse);
     constexpr int TR = 4 * KG, KR = 64 / TR;
     const int rr = threadIdx.x % kRows, tr = threadIdx.x / kRows;
     const float* ssp = (const float*)(a.frag + (size_t)min((row0 + rr) / kBM, last_tile) * tile_bytes + kSsOff) + (rr & (kBM - 1));
+    const int classes = min(L::kSquares, (nchunks + 63) / 64);
     float sq[KR];
-    if (norm) {
+    auto load_squares = [&](int first) {  // the chunks first.. of a class of 64 threads
 #pragma unroll
         for (int k = 0; k < KR; k++) {
-            const int c = tr + TR * k;
+            const int c = first + tr + TR * k;
             const float v = ssp[(size_t)min(c, nchunks - 1) * (kChunkBytes / 4)];
             sq[k] = c < nchunks ? v : 0.0f;
         }
-    }
+    };
+    if (norm) load_squares(0);
     for (int j = 0; j < min(kWideRing - 1, iters); j++)
 #pragma unroll
         for (int u = 0; u < kPer; u++) issue(j, j, u);
     if (norm) {
-        for (int c0n = 64; c0n < nchunks; c0n += 64)
+        for (int q = 0; q < classes; q++) {
+            if (q > 0) load_squares(64 * q);
+            for (int c0n = 64 * q + 256; c0n < nchunks; c0n += 256)
 #pragma unroll
-            for (int k = 0; k < KR; k++) {
-                const int c = c0n + tr + TR * k;
-                const float v = ssp[(size_t)min(c, nchunks - 1) * (kChunkBytes / 4)];
-                sq[k] += c < nchunks ? v : 0.0f;
-            }
+                for (int k = 0; k < KR; k++) {
+                    const int c = c0n + tr + TR * k;
+                    const float v = ssp[(size_t)min(c, nchunks - 1) * (kChunkBytes / 4)];
+                    sq[k] += c < nchunks ? v : 0.0f;
+                }
 #pragma unroll
-        for (int d = KR / 2; d >= 1; d >>= 1)
+            for (int d = KR / 2; d >= 1; d >>= 1)
 #pragma unroll
-            for (int k = 0; k < d; k++) sq[k] += sq[k + d];
-        lds.parts[tr * kRows + rr] = sq[0];
+                for (int k = 0; k < d; k++) sq[k] += sq[k + d];
+            lds.parts[q][tr * kRows + rr] = sq[0];
+        }
     }
     float16_t acc[2][2] = {};
     for (int b = 0; b < nmine; b += 16) {
@@ -323,14 +330,18 @@ __device__ __forceinline__ void wide_tile(const GemmArgs& a, WideLds<KG>& lds, c
     if (threadIdx.x < kRows) {
         float inv = 1.0f;
         if (norm) {
-            float t[TR];
+            float sum = 0.0f;
+            for (int q = 0; q < classes; q++) {
+                float t[TR];
 #pragma unroll
-            for (int k = 0; k < TR; k++) t[k] = lds.parts[k * kRows + threadIdx.x];
+                for (int k = 0; k < TR; k++) t[k] = lds.parts[q][k * kRows + threadIdx.x];
 #pragma unroll
-            for (int d = TR / 2; d >= 1; d >>= 1)
+                for (int d = TR / 2; d >= 1; d >>= 1)
 #pragma unroll
-                for (int k = 0; k < d; k++) t[k] += t[k + d];
-            inv = 1.0f / sqrtf(t[0] / (float)a.K + a.eps);
+                    for (int k = 0; k < d; k++) t[k] += t[k + d];
+                sum += t[0];
+            }
+            inv = 1.0f / sqrtf(sum / (float)a.K + a.eps);
         }
         sinv[threadIdx.x] = inv;
     }

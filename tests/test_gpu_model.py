@@ -185,6 +185,22 @@ def test_chunked_prefill_does_not_depend_on_the_chunking(pair):
     assert np.max(np.abs(a - m.logits())) < 1e-4 and ta == m.last_token()
 
 
+def test_chunked_prefill_of_a_wide_model_does_not_depend_on_the_chunking():
+    """The same for a hidden size above 4096 (more than 64 chunks of 64 columns): the in-projection of 576
+    rows applies its RMSNorm inside the GEMM, that of 64 rows in the reduce, from the same sums of x^2."""
+    cfg = dict(layers=2, full_attention_every=2, hidden=6144, intermediate=512, vocab=512, n_q_heads=2, n_kv_heads=1,
+               head_dim=256, gdn_heads=4)
+    index, buf = W.synth_model(cfg, seed=29, body="q4", head="f16", norm_jitter=0.1)
+    ids = prompt(cfg["vocab"], 576, 31)
+    with Q.Model.load(index, buf, options={"engine": "graph"}) as m:
+        m.prefill_chunk(ids, 0, True)
+        whole = m.logits()
+        m.reset()
+        for at in range(0, 576, 64):
+            m.prefill_chunk(ids[at:at + 64], at, at == 512)
+        assert np.all(np.isfinite(whole)) and np.array_equal(m.logits(), whole)
+
+
 def test_chunked_prefill_matches_oracle_over_many_chunks(pair):
     name, m, om, _, _ = pair
     ids = prompt(m.vocab, 1100, 12)  # one pass (passes hold up to 2048 tokens)
