@@ -102,7 +102,7 @@ class BatchDecoder {
     int32_t* order_ = nullptr;  // the step's rows by decreasing position (attention partials' order)
     void* am_scratch_ = nullptr;  // per-row argmax partials
     uint32_t* host_u32_ = nullptr;  // pinned, 2 * 64 entries
-    static constexpr int kReadSlots = 4;
+    static constexpr int kReadSlots = 8, kReadThreads = 4;
     static constexpr size_t kReadSlot = 2u << 20;
     uint8_t* host_read_ = nullptr;  // pinned, kReadSlots x kReadSlot bytes: logits on their way out
     hipEvent_t read_ev_[kReadSlots] = {};

@@ -14,6 +14,7 @@
 
 #include "error.hpp"
 #include "hip_util.hpp"
+#include "host_read.hpp"
 #include "json.hpp"
 #include "kernels/decode.hpp"
 #include "kernels/launch.hpp"
@@ -21,17 +22,11 @@
 namespace qne {
 
 void wait_stream(hipStream_t st, double timeout_s) {
-    using clk = std::chrono::steady_clock;
-    const auto start = clk::now();
-    int spins = 0;
-    while (true) {
-        hipError_t e = hipStreamQuery(st);
-        if (e == hipSuccess) return;
+    poll_device([st] {
+        const hipError_t e = hipStreamQuery(st);
         if (e != hipErrorNotReady) hip_check(e, "hipStreamQuery");
-        if (++spins > 2000) std::this_thread::sleep_for(std::chrono::microseconds(50));
-        if (std::chrono::duration<double>(clk::now() - start).count() > timeout_s)
-            throw Error(QNE_EDEVICE, "GPU wait failed: timed out after " + std::to_string((long long)timeout_s) + " s");
-    }
+        return e == hipSuccess;
+    }, timeout_s);
 }
 
 // ModelTiles::validate (kernels/src/model.rs:101-109) on a serialised tile profile: each of the six

@@ -276,6 +276,23 @@ def test_batch_continues_each_sequence_like_the_oracle(pair):
         assert got == want_ids[1:], r
 
 
+def test_batch_logits_of_many_rows_equal_those_of_few():
+    """40 rows of 32768 logits (three slots of the readback's ring, the last one ragged) against the same
+    rows four at a time, which are copied straight: a row's bits do not depend on the batch."""
+    cfg = dict(layers=1, full_attention_every=2, hidden=512, intermediate=512, vocab=32768, n_q_heads=2, n_kv_heads=1,
+               head_dim=256, gdn_heads=4)
+    index, buf = W.synth_model(cfg, seed=5, body="q4", head="f16")
+    tokens = np.random.default_rng(2).integers(0, cfg["vocab"], 40).astype(np.uint32)
+    with Q.Model.load(index, buf) as m, Q.Batch(m, max_rows=40, max_context=16) as b:
+        def logits(toks):
+            for r, t in enumerate(toks):
+                b.reset_row(r, int(t))
+            return b.step(len(toks), logits=True)[1]
+
+        few = np.concatenate([logits(tokens[i:i + 4]) for i in range(0, 40, 4)])
+        assert np.array_equal(logits(tokens), few)
+
+
 def test_batch_teacher_forced_logits_and_empty_rows(pair):
     """Rows started empty (reset_row) and fed given tokens: every step's logits against the
     oracle's token-by-token run from position 0."""
