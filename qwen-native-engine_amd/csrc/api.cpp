@@ -378,19 +378,22 @@ int qne_gemm(int kind, const void* w, const void* sz, int rows, int k, int group
         a.N = rows;
         a.K = k;
         a.group = kind == QNE_MAT_Q4 ? group : 64;
-        // up to 256 rows share one split count and form, so a row's sums do not depend on the call;
-        // longer calls would write a partial of every row per split and run as a prompt's pass
-        if (m > 256 && kind == QNE_MAT_Q4) a.row_tiles = (m + 63) / 64;
-        // (and at least 8 chunks a split: 400 x 100 x 2048 with two took 23 us)
-        a.splits = qne::gemm_splits(kind, rows, k, a.group, a.row_tiles);
-        if (a.row_tiles > 1) {
-            const int nch = k / 64, most = std::max(1, std::min(a.splits, nch / 8)), per = (nch + most - 1) / most;
-            a.splits = (nch + per - 1) / per;  // no empty split
-        }
         a.epi = epilogue;
         a.y = y;
         a.y_stride = y_stride;
         a.n_out = n_out;
+        // one split count and form for the matrix, so a row's sums do not depend on the call
+        a.splits = qne::gemm_splits(kind, rows, k, a.group);
+        // but above 256 rows that writes a partial of every row per split, and where it pays the call runs as
+        // a prompt's pass, with at least 8 chunks a split (400 x 100 x 2048 with two took 23 us)
+        if (m > 256 && kind == QNE_MAT_Q4) {
+            qne::GemmArgs pass = a;
+            pass.row_tiles = (m + 63) / 64;
+            const int nch = k / 64, fit = qne::gemm_splits(kind, rows, k, a.group, pass.row_tiles);
+            const int most = std::max(1, std::min(fit, nch / 8)), per = (nch + most - 1) / most;
+            pass.splits = (nch + per - 1) / per;  // no empty split
+            if (qne::gemm_wide_pays(pass)) a = pass;
+        }
         const size_t part = (size_t)a.splits * ((m + 63) / 64 * 64) * rows;
         const size_t frag = (qne::gemm_frag_bytes(k, m) + 255) / 256 * 256;
         const size_t szt = kind == QNE_MAT_Q4 ? qne::tile_sz_words(rows, k / a.group) : 0;

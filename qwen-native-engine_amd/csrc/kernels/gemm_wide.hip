@@ -635,6 +635,20 @@ bool gemm_is_short(const GemmArgs& a) {
     return wgs <= (a.m <= 128 ? 768 : 512);
 }
 
+// Calls of 257 to 2048 rows, N 64..12288, K 512..6144. A CU pays ~10 us for a pass's form before its matrix
+// units are busy, so it takes 5 of the 64-row form's 256 x 64 x 64 tile chunks a CU to be worth that (N x K
+// x rows, us, 64-row form / pass: 1847 x 640 x 502, 640 tile chunks, 25 / 29; 1557 x 1216 x 361, 798, 26 / 29;
+// 977 x 2816 x 445, 1232, 34 / 29; 442 x 5824 x 1489, 4368, 60 / 43), unless the pass saves the partials
+// too, one split with its own epilogue (3233 x 640 x 600, 1300, 39 / 24). Of 500 drawn calls (log-uniform)
+// 2 are over 1 % slower than the 64-row form with its staging in two launches (2 and 5 %); with passes
+// throughout a third were, by up to 1.4x.
+bool gemm_wide_pays(const GemmArgs& a) {
+    const int64_t tiles = (int64_t)((a.N + kWideCols - 1) / kWideCols) * a.row_tiles;
+    if (tiles * (a.K / kChunk) > 1344) return true;
+    const bool own = a.epi != EPI_SWIGLU || (a.n_out % (kWideCols / 2) == 0 && a.K <= 64 * kChunk);
+    return a.splits == 1 && own && !gemm_is_short(a);
+}
+
 void launch_gemm_wide(GemmArgs a, hipStream_t st) {
     const int cols = (a.N + kWideCols - 1) / kWideCols;
     a.wide_cols = gemm_wide_cols(a.N, a.row_tiles, a.splits);

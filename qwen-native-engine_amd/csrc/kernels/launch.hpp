@@ -232,6 +232,9 @@ void launch_gemm(GemmArgs a, hipStream_t st);
 // The GEMM of a pass over a prompt (gemm_wide.hip), called by launch_gemm with the epilogue decided.
 // A call of few rows (gemm_is_short) writes split partials only.
 bool gemm_is_short(const GemmArgs& a);
+// Whether a q4 call of many rows, with the splits and row tiles of a pass, is faster as one than in the
+// 64-row form.
+bool gemm_wide_pays(const GemmArgs& a);
 void launch_gemm_wide(GemmArgs a, hipStream_t st);
 // The tile-major copy of q4 (scale, zero) words the row-tiled GEMM reads (GemmArgs::SZT):
 // tile_sz_words(rows, groups) words.

@@ -224,6 +224,24 @@ def test_gemm_row_result_does_not_depend_on_other_rows():
     assert np.array_equal(big.numpy()[237], one.numpy()[0])
 
 
+@pytest.mark.parametrize("rows,k,M", [(753, 768, 822), (190, 1024, 1632), (660, 768, 1322), (1989, 1152, 295), (256, 64, 2048)])
+def test_gemm_of_a_small_matrix_keeps_its_form_above_256_rows(rows, k, M):
+    """Many rows of a matrix that a pass's form would not pay for (it took 1.1 to 1.2 times as long) run as
+    few rows do: row by row the same bits as calls of one row."""
+    rng = np.random.default_rng(M)
+    _, w, sz = q4_matrix(rows, k, 64, rng)
+    X = rng.normal(size=(M, k)).astype(np.float32)
+    dw, dsz, dx = to_dev(w), to_dev(sz), to_dev(X)
+    full, one = D.zeros((M, rows), np.float32), D.zeros((3, rows), np.float32)
+    Q.gemm(Q.MAT_Q4, dw.data_ptr(), dsz.data_ptr(), rows, k, 64, dx.data_ptr(), k, M, full.data_ptr(), rows)
+    picks = [0, 64 * (M // 128) + 3, M - 1]
+    for i, r in enumerate(picks):
+        Q.gemm(Q.MAT_Q4, dw.data_ptr(), dsz.data_ptr(), rows, k, 64, dx.data_ptr() + 4 * k * r, k, 1,
+               one.data_ptr() + 4 * rows * i, rows)
+    D.sync()
+    assert np.array_equal(full.numpy()[picks], one.numpy())
+
+
 def test_gemm_rejects_bad_shapes():
     for args in [(Q.MAT_F16, 0, 256, 1000, 4), (Q.MAT_Q4, 32, 256, 1024, 4), (Q.MAT_F16, 0, 256, 1024, 2049),
                  (Q.MAT_F16, 0, 256, 1024, 0)]:
