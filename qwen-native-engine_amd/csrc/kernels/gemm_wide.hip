@@ -61,8 +61,14 @@ struct Bf3 {
     }
 };
 
-// s (r - z): what the products of q - r leave of a group's zero point.
-__device__ __forceinline__ float zero_rest(uint32_t szw) { return lo_h(szw) * (zero_int(szw).value() - hi_h(szw)); }
+// s (r - z): what the products of q - r leave of a group's zero point (r as zero_int has it: both round
+// halves to even). The empty asm keeps the compiler from a branch around it where only some lanes want it.
+__device__ __forceinline__ float zero_rest(uint32_t szw) {
+    const float z = hi_h(szw);
+    float v = lo_h(szw) * (__builtin_amdgcn_fmed3f(rintf(z), 0.0f, 15.0f) - z);
+    asm volatile("" : "+v"(v));
+    return v;
+}
 
 constexpr int kWideCols = 256;  // W rows (output columns) of a workgroup
 constexpr int kWideWaves = 8;
@@ -217,8 +223,9 @@ __device__ __forceinline__ void wide_tile(const GemmArgs& a, WideLds<KG>& lds, c
             const bool live = b + 8 * hf + i < nmine;
 #pragma unroll
             for (int t = 0; t < 2; t++) {
+                const float rest = zero_rest(sz[t][i]);
                 xa[t].set(i, live ? xv[t][i] : 0.0f);
-                wb[t].set(i, live ? zero_rest(sz[t][i]) : 0.0f);
+                wb[t].set(i, live ? rest : 0.0f);
             }
         }
         if (b + 16 < nmine) load_sums(b + 16);
@@ -537,8 +544,9 @@ __global__ __launch_bounds__(64 * kWideWaves) void k_gemm_short(const GemmArgs a
 #pragma unroll
             for (int i = 0; i < 8; i++) {
                 const bool live = b + 8 * hf + i < nmine;
+                const float rest = zero_rest(sv[i]);
                 xa.set(i, live ? xv[i] : 0.0f);
-                wb.set(i, live ? zero_rest(sv[i]) : 0.0f);
+                wb.set(i, live ? rest : 0.0f);
             }
 #pragma unroll
             for (int p = 2; p >= 0; p--)

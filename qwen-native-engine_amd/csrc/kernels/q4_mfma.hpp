@@ -23,7 +23,6 @@ __device__ __forceinline__ uint32_t and_or(uint32_t v, uint32_t mask, uint32_t m
 // -64 - r, twice each. A sum of 1024 or more rounds to a whole number in f16, so z + 1024 is the rounding.
 struct ZeroInt {
     half2_t high, low;
-    __device__ __forceinline__ float value() const { return (float)high.x - 1024.0f; }
 };
 __device__ __forceinline__ ZeroInt zero_int(uint32_t szw) {
     const half2_t k1024 = {(_Float16)1024.0f, (_Float16)1024.0f}, k1039 = {(_Float16)1039.0f, (_Float16)1039.0f};
