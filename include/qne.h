@@ -192,7 +192,9 @@ int qne_paged_attn_decode_noalloc(const float* q, const float* k_new, const floa
  * into two f16 halves, so the products keep about 22 bits), with the same norm prologue and
  * epilogues as qne_gemv. The reference's 16-token GEMM (kernels/src/batch.rs:12-99, Gpu::gemm
  * lib.rs:341-347) generalised to M up to 2048 (in tiles of 64 rows). x rows at x + r * x_stride (x_stride >= k, a multiple of 4), y
- * rows at y + r * y_stride. k must be a multiple of 64 and q4 groups a multiple of 64. On the null
+ * rows at y + r * y_stride. k must be a multiple of 64 and q4 groups a multiple of 64. A row's result does
+ * not depend on the other rows' values; nor, bit for bit, on their number, for f16 weights and in calls of
+ * up to 256 rows. A q4 call of more rows may split k otherwise: the same precision, another rounding. On the null
  * stream the call returns when the result is ready. The split partials' scratch is kept per device
  * (grown when a call needs more): calls that overlap on one device must not be issued. */
 int qne_gemm(int kind, const void* w, const void* sz, int rows, int k, int group, const float* x,

@@ -36,10 +36,6 @@ namespace {
 
 using namespace lds_dma;
 
-__device__ __forceinline__ uint32_t pack_h2(float a, float b) {
-    return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)a) | ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)b) << 16);
-}
-
 }  // namespace
 
 // The x operand of a GEMM from f32 rows (x + r * x_stride; rows >= m are zero), times `gain` when set;

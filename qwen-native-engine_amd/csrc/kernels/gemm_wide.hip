@@ -19,12 +19,12 @@
 // chunk. 64 rows (KG = 2): 4 waves across, and the two halves of the workgroup take the even and the
 // odd chunks; their sums meet in LDS at the end. The second form gives matrices with few columns twice
 // the workgroups at the same LDS traffic per MFMA. Which form a column runs in depends on the matrix
-// and the caller's fixed row count, never on the rows of the call, so a row's sums are added in the
-// same order in every call.
+// and GemmArgs::row_tiles, never on the rows of the call beside them, so where a caller fixes row_tiles a
+// row's sums are added in the same order in every call.
 // Measured (2048 rows, K = 2048; before: the 64-row form of batch.hip at two workgroups per CU): N =
-// 12288 with its epilogue 257 -> 203 us (206 GFLOP of MFMA, 1.0 PFLOP/s; a loop of these MFMAs alone, on
-// such data, reaches 1.85: the card's power limit), N = 8224 186 -> 160 us, N = 2048 60 -> 43 us, N = 2048
-// over the 2B model's K (2048, 4096, 6144) 105 -> 75 us. What is left: a workgroup's start and end are
+// 12288 with its epilogue 257 -> 198 us (206 GFLOP of MFMA, 1.0 PFLOP/s; a loop of these MFMAs alone, on
+// such data, reaches 1.85: the card's power limit), N = 8224 186 -> 161 us, N = 2048 60 -> 43 us, N = 2048
+// over the 2B model's K (2048, 4096, 6144) 105 -> 76 us. What is left: a workgroup's start and end are
 // ~10 us with its CU's matrix units idle, and a chunk takes 1.7 us for 1.1 of MFMA. Without the DMAs, the
 // LDS reads and the vector work together the loop is 11 % faster. Measured and not kept: two 4-wave
 // workgroups of 64 x 256 on a CU (N = 12288: 305 us), the halves of a workgroup one phase apart (+5 %),

@@ -165,8 +165,10 @@ void launch_gdn_decode_rows(const float* proj, float* conv_state, const float* c
 // residual add, SwiGLU with n_out = N / 2); y may be null when frag_out is set. With frag_out the
 // result (times gain_out, column order order_out) is also staged as the next GEMM's x operand.
 // `part` holds splits * mpad * N floats (mpad: m rounded up to 64) unless the GEMM applies the
-// epilogue itself. The split count depends on the matrix only (gemm_splits), so a row's sums are
-// added in the same order whatever the number of rows.
+// epilogue itself. The split count and the form depend on the matrix and row_tiles only (gemm_splits), so
+// for one row_tiles a row's sums are added in the same order whatever the number of rows. The model's
+// passes and the batched step fix row_tiles once; qne_gemm has 1 up to 256 rows and, above, the call's own
+// where that pays (gemm_wide_pays).
 struct GemmArgs {
     const float* x = nullptr;
     int x_stride = 0;
@@ -224,8 +226,8 @@ void launch_sample(const SampleArgs& a, void* scratch, hipStream_t st);
 constexpr int kGemmRowsMax = 2048;
 size_t gemm_frag_bytes(int K, int m);
 // Split-K count of a GEMM on an N x K matrix: as many splits as keep a grid of N tiles x row_tiles
-// x splits within one workgroup per CU (at least 2 chunks per split, at most 24). A caller passes a
-// fixed row_tiles (not the rows of the call), so that a row's sums do not depend on the call.
+// x splits within one workgroup per CU (at least 2 chunks per split, at most 24). A caller whose row
+// results are not to depend on the call passes a fixed row_tiles (not the rows of the call).
 int gemm_splits(int kind, int N, int K, int group, int row_tiles = 1);
 bool gemm_shape_ok(int kind, int N, int K, int group, int m);
 void launch_gemm(GemmArgs a, hipStream_t st);
