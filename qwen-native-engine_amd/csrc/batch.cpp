@@ -412,9 +412,9 @@ void BatchDecoder::row_state(int n, uint32_t* tokens, uint32_t* pos) {
 // the runtime stages them through its own small buffer, with one thread that also takes the page faults
 // of a fresh destination. Here the transfers run through a ring of pinned slots and a few threads, which
 // end with the call, write the slots out while the next ones are in flight. Step with logits of 64 rows /
-// 16 / 8 of 608 KB: 5.9 / 2.26 / 1.85 ms straight, 3.3 / 2.04 / 1.85 through the ring (eight threads 3.5 /
-// 2.13 / 1.85), so up to two slots (6 rows: 1.79 / 1.82) go straight. Memory that the runtime knows (pinned,
-// managed) is copied to directly too. OMP_NUM_THREADS bounds the threads.
+// 32 / 16 / 8 of 608 KB: 5.8 / 3.0 / 2.3 / 1.84 ms straight, 3.7 / 2.65 / 2.1 / 1.82 through the ring; up to
+// two slots (6 rows) the threads cost what they save, so these go straight. Memory that the runtime knows
+// (pinned, managed) is copied to directly too. OMP_NUM_THREADS bounds the threads.
 void BatchDecoder::read_logits(int n, float* dst) {
     const size_t bytes = (size_t)n * m_.cfg_.vocab * 4;
     hipPointerAttribute_t at{};
